@@ -269,9 +269,15 @@ static bool pick_tile(int dim, int order, int physics, int *T) {
   return false;
 }
 
+// (groups hold these buffers and read both in every step: a mask set later
+// acts on them too)
 static int upload_tile_words(sem_mesh *m) {
   const TileSet &ts = m->tiles;
   if (!m->d_tile_words) SEM_TRY(dalloc(&m->d_tile_words, ts.words.size(), &m->tile_bytes));
+  if (!m->d_tile_slot) SEM_TRY(dalloc(&m->d_tile_slot, m->tile_slots.size(), &m->tile_bytes));
+  const bool dir = std::any_of(m->dirichlet.begin(), m->dirichlet.end(), [](uint8_t d) { return d != 0; });
+  for (uint32_t &w : m->tile_slots) w = dir ? w | kSlotDirichlet : w & ~kSlotDirichlet;
+  HIPCHK(hipMemcpyAsync(m->d_tile_slot, m->tile_slots.data(), m->tile_slots.size() * 4, hipMemcpyHostToDevice, m->stream));
   HIPCHK(hipMemcpyAsync(m->d_tile_words, ts.words.data(), ts.words.size() * 4, hipMemcpyHostToDevice, m->stream));
   HIPCHK(hipStreamSynchronize(m->stream));
   return 0;
@@ -284,7 +290,7 @@ static int upload_tile_words(sem_mesh *m) {
 // words in the same lattice order and share one table, which stays in the
 // caches: 4 bytes per slot less to read per tile and launch (one acoustic
 // shot, 10 of 73 KB at 4x4x2 tiles, 9 of 50 KB at 16x8).
-static int upload_tile_slots(sem_mesh *m) {
+static void number_tile_slots(sem_mesh *m) {
   TileSet &ts = m->tiles;
   const TileKernelInfo k = tile_kernel_info(m->dim, m->order, m->physics, ts.T);
   const int N = m->order, n = m->n, LX = ts.T[0] * N + 1, LY = ts.T[1] * N + 1;
@@ -313,10 +319,7 @@ static int upload_tile_slots(sem_mesh *m) {
       slot.push_back((uint32_t)(x + k.lxp * y + k.lxyp * z) | (in ? (uint32_t)(e * k.elem_stride + p) << 16 : 0u));
     }
   }
-  SEM_TRY(dalloc(&m->d_tile_slot, slot.size(), &m->tile_bytes));
-  HIPCHK(hipMemcpyAsync(m->d_tile_slot, slot.data(), slot.size() * 4, hipMemcpyHostToDevice, m->stream));
-  HIPCHK(hipStreamSynchronize(m->stream));
-  return 0;
+  m->tile_slots = std::move(slot);
 }
 
 void sem::free_tiles(sem_mesh *m) {
@@ -361,7 +364,7 @@ int sem::upload_tiles(sem_mesh *m) {
   const int dim = m->dim, nv = m->nv, npar = ref_npar(dim, m->physics), kp = kernel_npar(dim, m->physics);
   // padded tile element order (padding repeats element 0; never read)
   const int64_t E = (int64_t)ts.elem_order.size();
-  SEM_TRY(upload_tile_slots(m));
+  number_tile_slots(m);
   SEM_TRY(upload_tile_words(m));
   SEM_TRY(dalloc(&m->d_sh_part, ts.sh_part.size(), &m->tile_bytes));
   if (!ts.sh_part.empty())

@@ -289,7 +289,6 @@ int setup_group(sem_batch *b, int gi) {
   h.nsrc = g.nsrc;
   h.S = g.S;
   h.c = m->c;
-  h.has_dir = m->dirichlet.empty() ? 0 : 1;
   h.G = m->G;
   h.nsteps = g.nsteps;
   h.step = g.d_step;

@@ -24,6 +24,10 @@ constexpr uint32_t kNodeMask = (1u << 29) - 1;
 constexpr uint32_t kFlagDirichlet = 1u << 29;  // zero the stiffness row only
 constexpr uint32_t kFlagFirst = 1u << 30;      // first colour to touch the node: store
 constexpr uint32_t kFlagLast = 1u << 31;       // last colour: finalise (mass + Newmark)
+// Slot-table words of the tile kernel: LDS lattice slot, a flag set in every
+// word of a mesh that has Dirichlet nodes (only then are the words of a tile's
+// own nodes read for theirs), place of the total in the high half.
+constexpr uint32_t kSlotMask = 0x7fffu, kSlotDirichlet = 0x8000u;
 // Tile lattice slot outside the mesh (partial tile at the mesh edge).
 constexpr uint32_t kSlotEmpty = 0xffffffffu;
 
@@ -246,19 +250,18 @@ struct GroupDev {
   int32_t pad;
   // tile kernel (structured meshes): fields in tile-major node numbering
   const uint32_t *tile_words;   // per tile: own nodes, shared ones, padding
-  const uint32_t *tile_slot;    // slot tables, of each word: LDS lattice slot | place in the element results << 16
+  const uint32_t *tile_slot;    // slot tables, of each word: LDS lattice slot | kSlotDirichlet | place in the element results << 16
   const float *telem;     // per element in tile order: affine factors, then vertex material
   // coupled shots (fluid-solid pairs): external load added to a node's sum
   // at its first colour, null otherwise; a_ stored every step (the coupling
   // reads the velocities v = w - dt/2 a_ after each step)
   const float *ext;
   int32_t ap_always;
-  int32_t has_dir;  // the mesh has Dirichlet nodes
   // partial results of nodes shared by tiles or elements:
   // part[(s*c + comp)*part_stride + position]; the positions of the tiles'
   // shared words, or of every element node ([e][nd], like conn) with the list
   // of shared nodes
-  int32_t c, pad2;
+  int32_t c;
   int64_t part_stride;
   float *part;
   const int32_t *sh_part;
@@ -503,6 +506,7 @@ struct sem_mesh {
   sem::TileSet tiles;
   uint32_t *d_tile_words = nullptr;
   uint32_t *d_tile_slot = nullptr;
+  std::vector<uint32_t> tile_slots;  // its host copy
   int32_t *d_sh_part = nullptr;
   float *d_telem = nullptr, *d_mi_int = nullptr;
   int32_t *d_to_int = nullptr;  // DMPlex DOF -> internal node

@@ -204,7 +204,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
   const uint32_t own = W.own;
   const uint32_t s_end = W.s1;  // shots [s0, s1)
   const float gdt = G.dt;
-  const bool upd = !A.ku_only, has_dir = G.has_dir != 0, has_ext = G.ext != nullptr;
+  const bool upd = !A.ku_only, has_ext = G.ext != nullptr;
   const int64_t step = *glb(G.step) + A.koff;
   const bool over = step >= G.nsteps;
 
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
   // are coalesced.  Outside the column phase each thread writes and reads
   // only its own slots of su.
   // Per word: its LDS lattice slot and the place of its total in the element
-  // results (low and high half), and its inverse mass (own nodes) or
+  // results (low 15 bits and high half), and its inverse mass (own nodes) or
   // partial-result position (shared ones), kept for all the tile's shots.
   uint32_t slr[T::NIT], mik[T::NIT];
   constexpr int NRW = (ND + 63) / 64;
@@ -236,12 +236,16 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     const gptr<const uint32_t> slots = glb(G.tile_slot) + (int64_t)W.slots * T::NTL;
     const gptr<const uint32_t> gmi = (gptr<const uint32_t>)glb(G.mi) + own;
     const gptr<const uint32_t> gpos = (gptr<const uint32_t>)glb(G.sh_part) + W.sh_off;
-    uint32_t wv[T::NIT];  // node | Dirichlet flag
+    uint32_t wv[T::NIT];  // node | Dirichlet flag (own nodes: see kSlotDirichlet below)
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       const int k = min(tid + r * T::BT, T::NTL - 1);
       slr[r] = slots[k];
-      wv[r] = (k >= nint || has_dir) ? words[k] : own + k;
+      // (own nodes need no word; every lane loads all the same, those of the own
+      // nodes the first shared one: with a branch around it the compiler waits
+      // for each word before the next load, 64^3 acoustic hexes 202 -> 220 us)
+      const uint32_t word = words[max(k, min(nint, T::NTL - 1))];
+      wv[r] = k >= nint ? word : own + k;
       const gptr<const uint32_t> src = k < nint ? gmi + k : gpos + (min(k, nval - 1) - nint);
       mik[r] = nval > nint || k < nint ? *src : 0u;
     }
@@ -287,10 +291,14 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       if (tid + r * T::BT >= nval) continue;
-      const int l = slr[r] & 0xffffu;
+      const int l = slr[r] & kSlotMask;
       sw[l] = wv[r];
 #pragma unroll
       for (int c = 0; c < C; ++c) su[c * T::NTLP + l] = uv[r][c];
+    }
+    if (slr[0] & kSlotDirichlet) {
+#pragma unroll 1
+      for (int k = tid; k < nint; k += T::BT) sw[slots[k] & kSlotMask] = words[k];
     }
   }
 
@@ -570,7 +578,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       const bool ok = more && tid + r * T::BT < nval;
-      const uint32_t g = ok ? (sw[slr[r] & 0xffffu] & kNodeMask) : 0u;
+      const uint32_t g = ok ? (sw[slr[r] & kSlotMask] & kNodeMask) : 0u;
 #pragma unroll
       for (int c = 0; c < C; ++c) nu[r][c] = ok ? gu[((s + 1) * C + c) * GG + g] : 0.f;
     }
@@ -618,7 +626,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
       const int k = tid + r * T::BT;
       if (k >= nval) continue;
       const uint32_t sv = again(slr[r]);
-      const int l = sv & 0xffffu, o = sv >> 16;
+      const int l = sv & kSlotMask, o = sv >> 16;
 #pragma unroll
       for (int c = 0; c < C; ++c) {
         const float tot = sK[o + c * ND];
@@ -650,7 +658,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       if (tid + r * T::BT >= nval) continue;
-      const int l = slr[r] & 0xffffu;
+      const int l = slr[r] & kSlotMask;
 #pragma unroll
       for (int c = 0; c < C; ++c) su[c * T::NTLP + l] = nu[r][c];
     }
@@ -697,7 +705,7 @@ static bool same_shape(const int *T, int tx, int ty, int tz) {
 
 template <class S>
 static TileKernelInfo tile_info() {
-  static_assert(S::NTLP < 65536 && S::E * S::SKE < 65536, "LDS slots and result places are 16-bit");
+  static_assert(S::NTLP <= (int)kSlotMask && S::E * S::SKE < 65536, "LDS slots take 15 bits, result places 16");
   TileKernelInfo r{};
   r.lds_bytes = sizeof(float) * (size_t)S::LDS;
   r.threads = S::BT;
