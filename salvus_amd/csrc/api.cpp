@@ -179,11 +179,11 @@ int sem::ensure_pointwise(sem_mesh *m) {
 // that size a colour's launch runs for a hundred times its latency) and the
 // colours stay; so they do for a node of 63 elements or more (the classes are
 // counted on the device, one a lane; no mesh generator makes such a node).
+static std::mutex mesh_lazy;  // batches prepared in several threads may share a mesh
 constexpr double kMaxPartsPerNode = 1.6;
 constexpr int64_t kMaxSmallParts = (int64_t)256 << 20;
 int sem::ensure_elem_parts(sem_mesh *m) {
-  static std::mutex mu;  // batches prepared in several threads may share the mesh
-  std::lock_guard<std::mutex> lock(mu);
+  std::lock_guard<std::mutex> lock(mesh_lazy);
   if (m->elem_parts >= 0) return 0;
   // elements per node; the nodes of each count, block of nodes by block
   const int nb = (int)((m->G + kClassNodes - 1) / kClassNodes);
@@ -271,6 +271,7 @@ static bool pick_tile(int dim, int order, int physics, int *T) {
 
 // (groups hold these buffers and read both in every step: a mask set later
 // acts on them too)
+static void free_colour_tiles(sem_mesh *m);
 static int upload_tile_words(sem_mesh *m) {
   const TileSet &ts = m->tiles;
   if (!m->d_tile_words) SEM_TRY(dalloc(&m->d_tile_words, ts.words.size(), &m->tile_bytes));
@@ -290,25 +291,27 @@ static int upload_tile_words(sem_mesh *m) {
 // words in the same lattice order and share one table, which stays in the
 // caches: 4 bytes per slot less to read per tile and launch (one acoustic
 // shot, 10 of 73 KB at 4x4x2 tiles, 9 of 50 KB at 16x8).
-static void number_tile_slots(sem_mesh *m) {
-  TileSet &ts = m->tiles;
+static std::vector<uint32_t> number_tile_slots(const sem_mesh *m, const std::vector<uint16_t> &slot_of,
+                                               std::vector<int32_t> &table) {
+  const TileSet &ts = m->tiles;
+  table.resize(ts.ntiles);
   const TileKernelInfo k = tile_kernel_info(m->dim, m->order, m->physics, ts.T);
   const int N = m->order, n = m->n, LX = ts.T[0] * N + 1, LY = ts.T[1] * N + 1;
   const int64_t NTL = ts.slots_per_tile;
   std::vector<uint32_t> slot;
   std::map<std::tuple<int, int, int>, std::vector<int32_t>> tables;  // per tile extent: the first tile of each table
   for (int64_t t = 0; t < ts.ntiles; ++t) {
-    TileInfo &ti = ts.info[t];
+    const TileInfo &ti = ts.info[t];
     std::vector<int32_t> &seen = tables[std::make_tuple(ti.ex, ti.ey, ti.ez)];
-    const uint16_t *of = &ts.slot_of[t * NTL];
-    const auto same = [&](int32_t u) { return std::equal(of, of + NTL, &ts.slot_of[u * NTL]); };
+    const uint16_t *of = &slot_of[t * NTL];
+    const auto same = [&](int32_t u) { return std::equal(of, of + NTL, &slot_of[u * NTL]); };
     const auto it = std::find_if(seen.begin(), seen.end(), same);
     if (it != seen.end()) {
-      ti.slots = ts.info[*it].slots;
+      table[t] = table[*it];
       continue;
     }
     seen.push_back((int32_t)t);
-    ti.slots = (int32_t)(slot.size() / NTL);
+    table[t] = (int32_t)(slot.size() / NTL);
     for (int64_t i = 0; i < NTL; ++i) {
       const int l = of[i], x = l % LX, y = (l / LX) % LY, z = l / (LX * LY);
       const int a = std::min(x / N, ti.ex - 1), b = std::min(y / N, ti.ey - 1), c = std::min(z / N, ti.ez - 1);
@@ -319,10 +322,52 @@ static void number_tile_slots(sem_mesh *m) {
       slot.push_back((uint32_t)(x + k.lxp * y + k.lxyp * z) | (in ? (uint32_t)(e * k.elem_stride + p) << 16 : 0u));
     }
   }
-  m->tile_slots = std::move(slot);
+  return slot;
+}
+
+// Tables of the colour launches, built and uploaded once.
+int sem::ensure_colour_tiles(sem_mesh *m) {
+  std::lock_guard<std::mutex> lock(mesh_lazy);
+  ColourTiles &ct = m->ctiles;
+  if (ct.valid) return 0;
+  std::vector<uint16_t> slot_of;
+  build_colour_tiles(m, ct, slot_of);
+  ct.slots = number_tile_slots(m, slot_of, ct.table);
+  size_t bytes = 0;
+  auto up = [&](auto **dst, const auto &v) {
+    SEM_TRY(dalloc(dst, v.size(), &bytes));
+    if (v.empty()) return 0;
+    return hip_check(hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, m->stream), "upload");
+  };
+  int rc = up(&ct.d_words, ct.words);
+  if (!rc) rc = up(&ct.d_words_lat, ct.words_lat);
+  if (!rc) rc = up(&ct.d_slot, ct.slots);
+  if (!rc) rc = up(&ct.d_to_int, ct.to_internal);
+  if (!rc) rc = dalloc(&ct.d_mi, (size_t)m->G, &bytes);
+  if (!rc) rc = launch_permute_f32(m->G, ct.d_to_int, m->d_mi, ct.d_mi, m->stream);
+  if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
+  if (rc) {
+    free_colour_tiles(m);
+    return rc;
+  }
+  ct.valid = true;
+  m->tile_bytes += bytes;
+  m->bytes += bytes;
+  return 0;
+}
+
+static void free_colour_tiles(sem_mesh *m) {
+  ColourTiles &ct = m->ctiles;
+  dfree(ct.d_words);
+  dfree(ct.d_words_lat);
+  dfree(ct.d_slot);
+  dfree(ct.d_mi);
+  dfree(ct.d_to_int);
+  ct = ColourTiles();
 }
 
 void sem::free_tiles(sem_mesh *m) {
+  free_colour_tiles(m);
   dfree(m->d_tile_words);
   dfree(m->d_tile_slot);
   dfree(m->d_sh_part);
@@ -364,7 +409,11 @@ int sem::upload_tiles(sem_mesh *m) {
   const int dim = m->dim, nv = m->nv, npar = ref_npar(dim, m->physics), kp = kernel_npar(dim, m->physics);
   // padded tile element order (padding repeats element 0; never read)
   const int64_t E = (int64_t)ts.elem_order.size();
-  number_tile_slots(m);
+  {
+    std::vector<int32_t> table;
+    m->tile_slots = number_tile_slots(m, ts.slot_of, table);
+    for (int64_t t = 0; t < ts.ntiles; ++t) ts.info[t].slots = table[t];
+  }
   SEM_TRY(upload_tile_words(m));
   SEM_TRY(dalloc(&m->d_sh_part, ts.sh_part.size(), &m->tile_bytes));
   if (!ts.sh_part.empty())
@@ -442,6 +491,7 @@ static void mesh_free(sem_mesh *m) {
   dfree(m->d_telem);
   dfree(m->d_mi_int);
   dfree(m->d_to_int);
+  free_colour_tiles(m);
   if (m->stream) (void)hipStreamDestroy(m->stream);
   delete m;
 }
@@ -698,6 +748,17 @@ int sem_mesh_set_dirichlet(sem_mesh *m, const uint8_t *mask) {
       w = node | (dint[node] ? kFlagDirichlet : 0u);
     }
     SEM_TRY(upload_tile_words(m));
+    ColourTiles &ct = m->ctiles;
+    if (ct.valid) {
+      for (int64_t g = 0; g < m->G; ++g) dint[ct.to_internal[g]] = m->dirichlet[g];
+      for (auto *ws : {&ct.words, &ct.words_lat})
+        for (auto &w : *ws)
+          if (w != kSlotEmpty) w = (w & ~kFlagDirichlet) | (dint[w & kNodeMask] ? kFlagDirichlet : 0u);
+      HIPCHK(hipMemcpyAsync(ct.d_words, ct.words.data(), ct.words.size() * 4, hipMemcpyHostToDevice, m->stream));
+      if (ct.d_words_lat)
+        HIPCHK(hipMemcpyAsync(ct.d_words_lat, ct.words_lat.data(), ct.words_lat.size() * 4, hipMemcpyHostToDevice, m->stream));
+      HIPCHK(hipStreamSynchronize(m->stream));
+    }
   }
   return 0;
 }

@@ -22,7 +22,7 @@ int64_t field_pos(const Group &g, int64_t i) {
   if (!g.tiled) return i;
   const sem_mesh *m = g.mesh;
   const int64_t c = i / m->G, node = i - c * m->G;
-  return c * m->G + m->tiles.to_internal[node];
+  return c * m->G + (g.parts ? m->tiles.to_internal : m->ctiles.to_internal)[node];
 }
 
 void free_group(Group &g) {
@@ -62,11 +62,51 @@ int default_epb(int nd) {
   return best;
 }
 
+// SEM_TILE_OCCUPANCY=normal|high: the tile kernels of acoustic meshes run one
+// launch per colour, in the given variant (tests compare them).
+static const char *tile_occupancy(const sem_mesh *m) {
+  const char *e = m->physics == SEM_ACOUSTIC ? getenv("SEM_TILE_OCCUPANCY") : nullptr;
+  return e && (!strcmp(e, "high") || !strcmp(e, "normal")) ? e : nullptr;
+}
+
+// Whether the launch that a group's tiles join holds so many of them that one
+// launch per colour is faster (sets Group::heavy of `gi`).  With partial results
+// a step is one launch over all tiles, but its gathers and stores of shared
+// nodes cost bandwidth; with colours it is 8 launches, each with the latency
+// of its rounds of workgroups, on a numbering that leaves every tile fewer and
+// longer runs.  Measured on 3-D meshes (milliseconds a step with partial
+// results, with colours), by tile shots per workgroup that the chip holds:
+// 54: 4 shots of 48^3 elastic hexes 0.77, 0.85; 128: 4 of 64^3 1.72, 1.68, 8 of
+// 64^3 acoustic 1.37, 1.36; 163: 4 of 100^3 order-3 acoustic 1.09, 1.05; 182: 4 of
+// 72^3 2.57, 2.53; 216: 2 of 96^3 3.12, 2.81, 4 of 96^3 acoustic 2.34, 2.28; 256: 8
+// of 64^3 3.30, 3.08; 455: 8 of 128^3 order-2 acoustic 1.89, 1.89; 864: 8 of 96^3
+// 11.0, 10.1; 1280: 32 of 32^3 to 96^3 16.2, 14.6.  In 2-D (4 colours, few shared
+// nodes) the former colour kernel was slower at every size: 8 of 1000^2 elastic
+// 1.54, 1.71, 4 of 2000^2 acoustic 1.53, 1.78.
+constexpr int64_t kHeavyTiles = 160;
+static int weigh_group(sem_batch *b, int gi) {
+  Group &g = b->groups[gi];
+  const sem_mesh *m = g.mesh;
+  g.heavy = false;
+  if (b->path != SEM_PATH_FUSED || !m->tiles.valid || m->dim != 3) return 0;
+  int per_cu = 1, cus = 1;
+  SEM_TRY(tile_kernel_prepare(m->dim, m->order, m->physics, m->tiles.T, kTileParts, &per_cu));
+  HIPCHK(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device));
+  int64_t work = 0;
+  for (const Group &o : b->groups)
+    if (o.mesh->tiles.valid && o.mesh->dim == m->dim && o.mesh->order == m->order && o.mesh->physics == m->physics &&
+        std::equal(m->tiles.T, m->tiles.T + 3, o.mesh->tiles.T))
+      work += o.mesh->tiles.ntiles * o.S;
+  g.heavy = work >= kHeavyTiles * per_cu * cus;
+  return 0;
+}
+
 int setup_group(sem_batch *b, int gi) {
   Group &g = b->groups[gi];
   sem_mesh *m = g.mesh;
   const int path = b->path;
-  int rc = 0;
+  int rc = weigh_group(b, gi);
+  if (rc) return rc;
   // tile kernel: 32-bit field offsets, 16-bit shot numbers and at most
   // kTileMaxSrc sources per tile
   g.tiled = path == SEM_PATH_FUSED && m->tiles.valid &&
@@ -91,7 +131,8 @@ int setup_group(sem_batch *b, int gi) {
   // are read in each step) or the accumulator; kc = 0 is two bf16 zeros;
   // w = v + dt/2 a_ from the shot's initial v and a_
   if (path == SEM_PATH_FUSED && !g.tiled) SEM_TRY(ensure_elem_parts(m));
-  g.parts = g.tiled || (path == SEM_PATH_FUSED && m->elem_parts == 1 && g.S < 65536);
+  g.parts = g.tiled ? !(g.heavy || tile_occupancy(m)) : path == SEM_PATH_FUSED && m->elem_parts == 1 && g.S < 65536;
+  if (g.tiled && !g.parts) SEM_TRY(ensure_colour_tiles(m));
   const int64_t nparts = g.tiled ? m->tiles.nparts : m->nparts;
   SEM_TRY(dalloc(&g.fields, g.parts ? 4 * len + (size_t)g.S * m->c * nparts : 5 * len, &g.bytes));
   std::vector<float> buf;
@@ -187,7 +228,7 @@ int setup_group(sem_batch *b, int gi) {
       d.nodes_off = (int32_t)g.rec_nodes.size();
       for (int p = 0; p < m->nd; ++p) {
         const int32_t gid = m->conn[e * m->nd + p];
-        g.rec_nodes.push_back((uint32_t)(g.tiled ? m->tiles.to_internal[gid] : gid));
+        g.rec_nodes.push_back((uint32_t)field_pos(g, gid));
       }
       d.w_off = (int32_t)g.rec_w.size();
       d.shot = sl;
@@ -260,8 +301,9 @@ int setup_group(sem_batch *b, int gi) {
   GroupDev h{};
   h.conn = m->d_conn;
   if (g.tiled) {
-    h.tile_words = m->d_tile_words;
-    h.tile_slot = m->d_tile_slot;
+    h.tile_words = g.parts ? m->d_tile_words : m->ctiles.d_words;
+    h.tile_words_lat = m->ctiles.d_words_lat;
+    h.tile_slot = g.parts ? m->d_tile_slot : m->ctiles.d_slot;
     h.telem = m->d_telem;
     h.sh_part = m->d_sh_part;
   }
@@ -276,7 +318,7 @@ int setup_group(sem_batch *b, int gi) {
   h.geo_e = m->d_geo_e;
   h.par_e = m->d_par_e;
   h.geo_p = m->d_geo_p;
-  h.mi = g.tiled ? m->d_mi_int : m->d_mi;
+  h.mi = !g.tiled ? m->d_mi : g.parts ? m->d_mi_int : m->ctiles.d_mi;
   h.u = g.fields;
   h.w = g.fields + len;
   h.ap = g.fields + 2 * len;
@@ -416,6 +458,51 @@ static std::vector<TileItem> tile_items(sem_batch *b, const std::vector<int> &gi
   return items;
 }
 
+// Items of the launch of one tile colour: a tile each, with every shot of its
+// group.
+static std::vector<TileItem> colour_items(const sem_batch *b, const std::vector<int> &gis, int colour) {
+  std::vector<TileItem> items;
+  for (int gi : gis) {
+    const Group &g = b->groups[gi];
+    const sem_mesh *m = g.mesh;
+    for (int64_t t = 0; t < m->tiles.ntiles; ++t) {
+      const TileInfo &ti = m->tiles.info[t];
+      if (ti.colour != colour) continue;
+      const auto src = std::equal_range(g.tile_src.begin(), g.tile_src.end(), (int32_t)t);
+      TileItem it{};
+      it.group = gi;
+      it.tile = (int32_t)t;
+      it.s1 = (uint16_t)g.S;
+      it.ex = (uint8_t)ti.ex;
+      it.ey = (uint8_t)ti.ey;
+      it.ez = (uint8_t)ti.ez;
+      it.slots = m->ctiles.table[t];
+      it.src = (int32_t)(src.first - g.tile_src.begin());
+      it.nsrc = (int32_t)(src.second - src.first);
+      items.push_back(it);
+    }
+  }
+  return items;
+}
+
+// Acoustic colour launches take the high-occupancy variant when it needs fewer
+// rounds of workgroups over the CUs and a workgroup takes at most two shots: one
+// of its workgroups runs about 1.2x as long as a normal one, more with the
+// later shots, whose lattices it gathers in lattice order (ms a step normal, high:
+// one shot of 128^3 1.50, 1.43; two of 112^3 1.96, 1.90; four of 96^3 2.28, 2.38;
+// of 128^3 5.14, 5.35).  Both variants do the same arithmetic in the same order:
+// results are identical.
+static int colour_mode(const LaunchSet &L, const char *forced, int shots, int cus, int *mode) {
+  int lo = 1, hi = 1;
+  SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, kTileColours, &lo));
+  *mode = kTileColours;
+  if (L.physics != SEM_ACOUSTIC) return 0;
+  SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, kTileColoursHigh, &hi));
+  const auto rounds = [&](int64_t per_cu) { return (L.nitems + per_cu * cus - 1) / (per_cu * cus); };
+  if (forced ? !strcmp(forced, "high") : shots <= 2 && 6 * rounds(hi) < 5 * rounds(lo)) *mode = kTileColoursHigh;
+  return 0;
+}
+
 // Items of the shared-node launch behind it: 256 nodes of one class each, for
 // every plane (shot and component) of the group where that leaves enough
 // workgroups to fill the chip, else one item per plane; 512 nodes where there
@@ -545,7 +632,7 @@ static int build_plan(sem_batch *b) {
     sem_mesh *m = b->groups[gi].mesh;
     const bool t = b->groups[gi].tiled;
     const int shape = t ? m->tiles.T[0] * 10000 + m->tiles.T[1] * 100 + m->tiles.T[2] : 0;
-    const int tk = t ? 1 + 2 * (int)(m->tile_diag && !general) : b->groups[gi].parts ? 0 : 4;
+    const int tk = (t ? 1 + 2 * (int)(m->tile_diag && !general) : 0) + (b->groups[gi].parts ? 0 : 4);
     keys[std::make_tuple(lane[gi], tk, m->dim, m->order, m->physics, geo_mode(m), shape)].push_back(gi);
   }
   for (auto &l : b->launches) {
@@ -584,18 +671,29 @@ static int build_plan(sem_batch *b) {
     L.T[0] = shape / 10000;
     L.T[1] = (shape / 100) % 100;
     L.T[2] = shape % 100;
-    if (std::get<1>(kv.first) != 4) {
+    const bool colours = (std::get<1>(kv.first) & 4) != 0;
+    if (!colours) {
       auto &sg = shared[L.lane];
       sg.insert(sg.end(), kv.second.begin(), kv.second.end());
     }
-    if (L.kind == kLaunchTile) {
+    if (L.kind == kLaunchTile && colours) {
+      int shots = 1;
+      for (int gi : kv.second) shots = std::max(shots, b->groups[gi].S);
+      for (int c = 0; c < (1 << L.dim); ++c) {
+        const std::vector<TileItem> items = colour_items(b, kv.second, c);
+        L.colour = c;
+        L.nitems = (int)items.size();
+        SEM_TRY(colour_mode(L, tile_occupancy(b->groups[kv.second[0]].mesh), shots, cus, &L.mode));
+        if (!items.empty()) SEM_TRY(upload(&add(L)->d_tiles, items));
+      }
+    } else if (L.kind == kLaunchTile) {
       int per_cu = 1;
-      SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, &per_cu));
+      SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, kTileParts, &per_cu));
       const int waves = tile_kernel_info(L.dim, L.order, L.physics, L.T).threads / 64;
       const std::vector<TileItem> items = tile_items(b, kv.second, per_cu * cus, waves);
       L.nitems = (int)items.size();
       SEM_TRY(upload(&add(L)->d_tiles, items));
-    } else if (std::get<1>(kv.first) == 0) {
+    } else if (!colours) {
       std::vector<int32_t> elems;
       const int threads = block_threads(L.nd, b->epb);
       const std::vector<WorkItem> items = element_items(b, kv.second, 2048 / threads * cus, threads / 64, elems);
@@ -629,11 +727,11 @@ static int build_plan(sem_batch *b) {
   // launches of one step that kernel timing counts: tile and element launches
   // (a tile launch with the shared-node launch behind it), those of the same
   // kernel and colour in different lanes, which run side by side, once
-  std::set<std::tuple<int, int, int, int, int, int, int, int>> per_step;
+  std::set<std::tuple<int, int, int, int, int, int, int, int, bool>> per_step;
   for (const auto &L : b->launches)
     if (L.kind != kLaunchShared)
       per_step.insert(std::make_tuple((int)L.kind, (int)L.diag, L.dim, L.order, L.physics, L.gmode,
-                                      L.T[0] * 10000 + L.T[1] * 100 + L.T[2], L.colour));
+                                      L.T[0] * 10000 + L.T[1] * 100 + L.T[2], L.colour, L.mode != kTileParts));
   b->step_launches = (int)per_step.size();
   HIPCHK(hipStreamSynchronize(b->stream));
   return 0;
@@ -778,7 +876,7 @@ int enqueue_fused_step(sem_batch *b, int koff, int ku_only, int last) {
     a.ap_koff = last;
     a.pad = 0;
     auto go = [&]() {
-      if (L.kind == kLaunchTile) return launch_tile(L.dim, L.order, L.physics, L.T, L.diag, a, st);
+      if (L.kind == kLaunchTile) return launch_tile(L.dim, L.order, L.physics, L.T, L.diag, L.mode, a, st);
       if (L.kind == kLaunchShared) return launch_shared(a, st);
       return launch_fused(L.dim, L.order, L.physics, L.gmode, L.nitems, b->epb, L.nd, L.c, a, st);
     };
@@ -1146,7 +1244,7 @@ int sem_shot_get_field(sem_batch *b, int shot, int which, double *vals) {
   const float *ap = which == 1 ? field_base(b, *s, 2) + (size_t)s->slot * len : nullptr;  // v = w - dt/2 a_
   for (size_t i = 0; i < len; i += cap) {
     const size_t n = std::min(cap, len - i);
-    SEM_TRY(launch_read_field((int64_t)n, (int64_t)i, s->mesh->G, g.tiled ? s->mesh->d_to_int : nullptr, f, ap,
+    SEM_TRY(launch_read_field((int64_t)n, (int64_t)i, s->mesh->G, !g.tiled ? nullptr : g.parts ? s->mesh->d_to_int : s->mesh->ctiles.d_to_int, f, ap,
                               0.5 * g.dt, out, b->stream));
     HIPCHK(hipMemcpyAsync(vals + i, out, n * 8, hipMemcpyDeviceToHost, b->stream));
   }

@@ -68,7 +68,8 @@ struct Group {
   int nsrc = 0;
   std::vector<int32_t> tile_src;  // tiled: tile of each source, ascending
   bool tiled = false;       // tile kernel; fields in the mesh's tile-major numbering
-  bool parts = false;       // partial results at shared nodes (tiled, or element kernel without colours)
+  bool parts = false;       // partial results at shared nodes; else colour launches
+  bool heavy = false;       // of a batch whose tiles fill the chip often enough for colour launches
   int64_t *d_step = nullptr;  // device step counter
   float *d_seis = nullptr;    // seismograms of the group's shots
   int64_t seis_len = 0;
@@ -119,6 +120,7 @@ struct LaunchSet {
   int dim, order, physics, nd, c, colour;
   int gmode;  // geometry mode of the element kernel (kGeo*)
   bool diag;  // tile kernel: diagonal-geometry variant
+  int mode;   // tile kernel: kTileParts, kTileColours or kTileColoursHigh
   int nitems;
   int T[3];  // tile shape (tile kernel)
   int lane;  // stream lane (0: the batch stream, 1: the second stream)
@@ -185,6 +187,8 @@ int ensure_pointwise(sem_mesh *m);
 // Decides (once) whether the element kernel keeps partial results on this mesh
 // and builds their classes and positions.
 int ensure_elem_parts(sem_mesh *m);
+// Builds (once) what colour launches over the mesh's tiles need.
+int ensure_colour_tiles(sem_mesh *m);
 // noalloc.cpp: what the allocation-free operator keeps with a small mesh.
 int setup_apply(sem_mesh *m);
 int locate(const sem_mesh *m, const double *pt, int64_t *elem, double *ref);

@@ -249,7 +249,8 @@ struct GroupDev {
   int32_t quirks;
   int32_t pad;
   // tile kernel (structured meshes): fields in tile-major node numbering
-  const uint32_t *tile_words;   // per tile: own nodes, shared ones, padding
+  const uint32_t *tile_words;   // per tile: own nodes, shared ones, padding (colours: in node order, with flags)
+  const uint32_t *tile_words_lat;  // the same in lattice order (high-occupancy colour launches)
   const uint32_t *tile_slot;    // slot tables, of each word: LDS lattice slot | kSlotDirichlet | place in the element results << 16
   const float *telem;     // per element in tile order: affine factors, then vertex material
   // coupled shots (fluid-solid pairs): external load added to a node's sum
@@ -321,6 +322,20 @@ struct TileSet {
   std::vector<int32_t> to_internal;  // DMPlex DOF -> internal node
   std::vector<int32_t> elem_order;   // tile-order position -> element (-1: padding)
   std::vector<int32_t> elem_pos;     // element -> tile-order position
+};
+
+// The tables of the colour launches over the same tiles (build_colour_tiles), in
+// a node numbering of their own.
+struct ColourTiles {
+  bool valid = false;
+  std::vector<uint32_t> words;       // per tile, in node order: node | flags, or kSlotEmpty
+  std::vector<uint32_t> words_lat;   // acoustic: the same words in lattice order
+  std::vector<int32_t> table;        // slot table of each tile
+  std::vector<uint32_t> slots;
+  std::vector<int32_t> to_internal;  // DMPlex DOF -> node
+  uint32_t *d_words = nullptr, *d_words_lat = nullptr, *d_slot = nullptr;
+  float *d_mi = nullptr;
+  int32_t *d_to_int = nullptr;
 };
 
 // Kernel argument blocks (passed by value; recorded by graph capture).
@@ -430,6 +445,10 @@ int launch_read_field(int64_t n, int64_t i0, int64_t G, const int32_t *to, const
 int launch_advance(int ngroups, const GroupDev *groups, int64_t k, hipStream_t st);
 
 // ---------------------------------------------------------------- tile kernel (tile_kernels.hip)
+// Modes of the tile kernel: every tile in one launch, partial results at nodes
+// shared by tiles; one launch per tile colour, sums of shared nodes in HBM; the
+// same with more waves per SIMD (acoustic).
+enum { kTileParts, kTileColours, kTileColoursHigh };
 int init_tile_tables(int device);
 struct TileKernelInfo {
   size_t lds_bytes;  // 0: no kernel compiled for this order and tile shape
@@ -440,10 +459,11 @@ struct TileKernelInfo {
 TileKernelInfo tile_kernel_info(int dim, int order, int physics, const int *T);
 // Compiled tile shapes for (dim, order, physics): up to max triples; returns the count.
 int tile_kernel_shapes(int dim, int order, int physics, int *shapes, int max);
-// Readies the kernel of this shape (LDS limit) and returns its workgroups per CU.
-int tile_kernel_prepare(int dim, int order, int physics, const int *T, int *per_cu);
+// Readies the kernel of this shape and mode (LDS limit) and returns its workgroups per CU.
+int tile_kernel_prepare(int dim, int order, int physics, const int *T, int mode, int *per_cu);
 // One workgroup per item (a.tiles).
-int launch_tile(int dim, int order, int physics, const int *T, bool diag, const FusedArgs &a, hipStream_t st);
+int launch_tile(int dim, int order, int physics, const int *T, bool diag, int mode, const FusedArgs &a,
+                hipStream_t st);
 
 // Bins over the elements' bounding boxes: the elements whose box meets bin b
 // are elem[start[b] .. start[b + 1]), ascending.
@@ -510,6 +530,7 @@ struct sem_mesh {
   int32_t *d_sh_part = nullptr;
   float *d_telem = nullptr, *d_mi_int = nullptr;
   int32_t *d_to_int = nullptr;  // DMPlex DOF -> internal node
+  sem::ColourTiles ctiles;  // built by the first group that takes colour launches
   bool tile_diag = false;  // every element's affine factors diagonal (axis-aligned lattice)
   size_t bytes = 0;       // device bytes held (tile path included)
   size_t tile_bytes = 0;  // of which the tile path
@@ -535,4 +556,6 @@ inline int pointwise_mode(const sem_mesh *m) {
 }
 // Tiles a logically Cartesian mesh; 0 = tiled, 1 = not eligible.
 int build_tiles(sem_mesh *m, int Tx, int Ty, int Tz, TileSet &ts);
+// Numbering, words and lattice slot of each word (slot_of) for colour launches.
+void build_colour_tiles(const sem_mesh *m, ColourTiles &ct, std::vector<uint16_t> &slot_of);
 }  // namespace sem

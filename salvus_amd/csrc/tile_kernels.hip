@@ -31,18 +31,19 @@
 //           that a_ is only written).
 // One launch over every tile, instead of one per tile colour with nodes
 // finished by the last colour, fills the chip and takes one latency chain per
-// step instead of 4 (2-D) or 8 (3-D); the partial results cost 12 % more
-// traffic in 3-D (elastic 4x2x2 tiles) and 4 % in 2-D.  Measured per step,
-// one MI355X, colours -> now: 100^2 acoustic quads 33 -> 11.7 us, 4 shots of
-// 331x287 acoustic quads 92 -> 39.7 us, 500^2 elastic quads 67 -> 52 us, 64^3
-// acoustic hexes 281 -> 202 us, 27x25x23 elastic hexes of order 3 78 -> 24 us,
-// 8 shots of 32^3 elastic hexes 482 -> 451 us, 4 shots of 64^3 1831 -> 1798 us
-// (there HBM runs at 3.5 of the 4.7 TB/s of a copy in k_tile and at 4.3 in
-// k_shared, and the VALU is 62 % busy: two 128-register workgroups a CU).  In
-// the largest batches the extra traffic costs more than the launches did: 32
-// shots of 32^3 to 96^3 16.1 -> 16.9 ms, 8 shots of 96^3 10.8 -> 11.3, but one
-// and two shots of 96^3 1.71 -> 1.54 and 3.09 -> 3.02, one acoustic shot of
-// 128^3 1.55 -> 1.52.
+// step instead of 4 (2-D) or 8 (3-D).  Measured per step, one MI355X, colours ->
+// now: 100^2 acoustic quads 33 -> 10.1 us, 4 shots of 331x287 acoustic quads 97 ->
+// 39 us, 500^2 elastic quads 70 -> 52 us, 64^3 acoustic hexes 285 -> 202 us,
+// 27x25x23 elastic hexes of order 3 78 -> 24 us, 8 shots of 32^3 elastic hexes
+// 486 -> 456 us, 4 shots of 64^3 1833 -> 1808 us (there HBM runs at 3.5 of the 4.7
+// TB/s of a copy in k_tile and at 4.3 in k_shared, and the VALU is 62 % busy: two
+// 128-register workgroups a CU).  In large 3-D batches the launches' latencies
+// matter no more and the scattered shared nodes cost bandwidth (k_tile 3.6 TB/s
+// against 4.2): there the tiles run one launch per colour (MODE), on a node
+// numbering of its own in which the tile that finishes a node holds it, with
+// the sums of shared nodes in HBM between the colours; batch.cpp says from
+// which size on.  32 shots of 32^3 to 96^3 elastic hexes: one launch 17.49 ms,
+// colours 16.11.
 // The operator is the one of TensorQuad.cpp:176-210/:350-397 and
 // Hexahedra.cpp:579-754 (sum-factorised gradient, J^-T contraction,
 // test-and-integrate) with Scalar.cpp:42-71, Elastic2D.cpp:53-82 and
@@ -165,12 +166,17 @@ __device__ __forceinline__ float p1_face(int v, float a, float b) {
 // diagonal (axis-aligned lattices), so the contractions keep their diagonal
 // terms only; the terms dropped are exact zeros, so results are those of the
 // general kernel.
-template <int DIM, int N, int PHYS, int TX, int TY, int TZ, bool DG>
-__global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
-    __attribute__((amdgpu_waves_per_eu(TS<DIM, N, PHYS, TX, TY, TZ>::MINW))) k_tile(FusedArgs A) {
-  using T = TS<DIM, N, PHYS, TX, TY, TZ>;
+// MODE: partial results at shared nodes, or one launch per tile colour with the
+// sums of shared nodes in HBM (kTileColours; kTileColoursHigh: its acoustic
+// high-occupancy variant).
+template <int DIM, int N, int PHYS, int TX, int TY, int TZ, bool DG, int MODE>
+__global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ, MODE == kTileColoursHigh>::BT))
+    __attribute__((amdgpu_waves_per_eu(TS<DIM, N, PHYS, TX, TY, TZ, MODE == kTileColoursHigh>::MINW)))
+    k_tile(FusedArgs A) {
+  constexpr bool COL = MODE != kTileParts, HO = MODE == kTileColoursHigh;
+  using T = TS<DIM, N, PHYS, TX, TY, TZ, HO>;
   constexpr int n = T::n, C = T::C, ND = T::ND, NL = T::NL;
-  static_assert(T::NIT == T::KF, "every slot's finish inputs are loaded ahead");
+  static_assert(HO || T::NIT == T::KF, "every slot's finish inputs are loaded ahead");
   extern __shared__ float lds[];
   float *su = lds;
   uint32_t *sw = reinterpret_cast<uint32_t *>(lds + T::O_SW);
@@ -194,7 +200,9 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
   const gptr<float> gw = glb(G.w);
   const gptr<float> gap = glb(G.ap);
   const gptr<uint32_t> gkc = glb(G.kc);
-  const gptr<float> gpart = glb(G.part);
+  const gptr<float> gpart = glb(G.part), gacc = glb(G.acc);
+  const gptr<const float> gext = glb(G.ext);
+  const gptr<const uint32_t> gmi = (gptr<const uint32_t>)glb(G.mi);
   const int64_t PS = G.part_stride;
   const uint32_t GG = (uint32_t)G.G;
   const int ex = W.ex, ey = W.ey, ez = W.ez;
@@ -226,28 +234,39 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
   // Per word: its LDS lattice slot and the place of its total in the element
   // results (low 15 bits and high half), and its inverse mass (own nodes) or
   // partial-result position (shared ones), kept for all the tile's shots.
-  uint32_t slr[T::NIT], mik[T::NIT];
+  // (High occupancy: the words come in lattice order, so slots need no table,
+  // and inverse masses are read with the other finish inputs.)
+  uint32_t slr[HO ? 1 : T::NIT], mik[HO ? 1 : T::NIT];
+  const auto slot = [&](int r) {  // (colours: -1 past the end)
+    const int k = tid + r * T::BT;
+    if constexpr (HO) return k < T::NTL ? T::lds_slot(k) : -1;
+    else return COL && k >= T::NTL ? -1 : (int)(slr[r] & kSlotMask);
+  };
   constexpr int NRW = (ND + 63) / 64;
   float rw[NRW];
   int rec_c = -1, rec_e = 0;
   gptr<float> rec_out = nullptr;
   {
-    const gptr<const uint32_t> words = glb(G.tile_words) + (int64_t)W.tile * T::NTL;
+    const gptr<const uint32_t> words = glb(HO ? G.tile_words_lat : G.tile_words) + (int64_t)W.tile * T::NTL;
     const gptr<const uint32_t> slots = glb(G.tile_slot) + (int64_t)W.slots * T::NTL;
-    const gptr<const uint32_t> gmi = (gptr<const uint32_t>)glb(G.mi) + own;
     const gptr<const uint32_t> gpos = (gptr<const uint32_t>)glb(G.sh_part) + W.sh_off;
-    uint32_t wv[T::NIT];  // node | Dirichlet flag (own nodes: see kSlotDirichlet below)
+    uint32_t wv[T::NIT];  // node | flags (own nodes: see kSlotDirichlet below)
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       const int k = min(tid + r * T::BT, T::NTL - 1);
-      slr[r] = slots[k];
-      // (own nodes need no word; every lane loads all the same, those of the own
-      // nodes the first shared one: with a branch around it the compiler waits
-      // for each word before the next load, 64^3 acoustic hexes 202 -> 220 us)
-      const uint32_t word = words[max(k, min(nint, T::NTL - 1))];
-      wv[r] = k >= nint ? word : own + k;
-      const gptr<const uint32_t> src = k < nint ? gmi + k : gpos + (min(k, nval - 1) - nint);
-      mik[r] = nval > nint || k < nint ? *src : 0u;
+      if constexpr (COL) {
+        wv[r] = tid + r * T::BT < T::NTL ? words[k] : kSlotEmpty;
+        if constexpr (!HO) slr[r] = slots[k];
+      } else {
+        slr[r] = slots[k];
+        // (own nodes need no word; every lane loads all the same, those of the own
+        // nodes the first shared one: with a branch around it the compiler waits
+        // for each word before the next load, 64^3 acoustic hexes 202 -> 220 us)
+        const uint32_t word = words[max(k, min(nint, T::NTL - 1))];
+        wv[r] = k >= nint ? word : own + k;
+        const gptr<const uint32_t> src = k < nint ? gmi + own + k : gpos + (min(k, nval - 1) - nint);
+        mik[r] = nval > nint || k < nint ? *src : 0u;
+      }
     }
     constexpr int NEI = (T::E * T::NED + T::BT - 1) / T::BT;
     static_assert(n * n <= T::BT && kTileMaxSrc <= T::BT, "staged one entry per thread");
@@ -258,8 +277,8 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     const float dv = TT.D[min(tid, n * n - 1)];
     // receivers of this item (one-shot items only, one wave per receiver
     // component): their weights come with the staging loads
-    rec_c = (tid >> 6) < W.nrec * C && A.koff > 0 && upd ? (tid >> 6) % C : -1;
-    if (rec_c >= 0) {
+    if (!COL) rec_c = (tid >> 6) < W.nrec * C && A.koff > 0 && upd ? (tid >> 6) % C : -1;
+    if (!COL && rec_c >= 0) {
       const TileRec R = glb(G.rec)[W.rec + (tid >> 6) / C];
       const gptr<const float> w = glb(G.rec_w) + R.w_off;
 #pragma unroll
@@ -268,6 +287,11 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
       rec_out = glb(R.out) + (step - 1) * R.stride + rec_c;
     }
     float uv[T::NIT][C];
+    if constexpr (COL && !HO) {
+#pragma unroll
+      for (int r = 0; r < T::NIT; ++r)
+        mik[r] = wv[r] != kSlotEmpty && (wv[r] & kFlagLast) && upd ? gmi[wv[r] & kNodeMask] : 0u;
+    }
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
       const uint32_t g = wv[r] == kSlotEmpty ? own : (wv[r] & kNodeMask);
@@ -290,13 +314,13 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     }
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
-      if (tid + r * T::BT >= nval) continue;
-      const int l = slr[r] & kSlotMask;
+      if (COL ? slot(r) < 0 : tid + r * T::BT >= nval) continue;
+      const int l = slot(r);
       sw[l] = wv[r];
 #pragma unroll
       for (int c = 0; c < C; ++c) su[c * T::NTLP + l] = uv[r][c];
     }
-    if (slr[0] & kSlotDirichlet) {
+    if (!COL && (slr[0] & kSlotDirichlet)) {
 #pragma unroll 1
       for (int k = tid; k < nint; k += T::BT) sw[slots[k] & kSlotMask] = words[k];
     }
@@ -318,7 +342,7 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
 
   // ---- receivers in this tile: su holds u after the previous step of the
   // block, sampled as k_receivers samples it (the same lanes and butterfly)
-  if (rec_c >= 0) {
+  if (!COL && rec_c >= 0) {
     const int ln = tid & 63;
     const int ea = rec_e % TX, eb = (rec_e / TX) % TY, ec3 = DIM == 3 ? rec_e / (TX * TY) : 0;
     const float *ue = su + rec_c * T::NTLP + ea * N + T::LXP * (eb * N) + (DIM == 3 ? T::LXYP * (ec3 * N) : 0);
@@ -560,25 +584,46 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     // ---- the own nodes' finish inputs (w = v + dt/2 a_ and the
     // compensations) and the next shot's lattice are loaded here so that
     // their latency overlaps the face passes
-    float vw[T::NIT][C];
-    uint32_t kc[T::NIT][C];
-#pragma unroll
-    for (int r = 0; r < T::NIT; ++r) {
-      const int k = tid + r * T::BT;
-      const bool fin = upd && k < nint;
+    // (colours: a node's sum so far too, for the first KF slots)
+    constexpr int KF = HO ? T::KF : T::NIT;
+    float vw[KF][C], prev[COL ? KF : 1][C];
+    uint32_t kc[KF][C], mia[HO ? KF : 1];
+    const auto load_slot = [&](int l, float(&p)[C], float(&w)[C], uint32_t(&q)[C], uint32_t *mi) {
+      const uint32_t word = l >= 0 ? sw[l] : kSlotEmpty;
+      const bool valid = word != kSlotEmpty;
+      const uint32_t g = valid ? word & kNodeMask : 0u;
+      const bool fin = valid && (word & kFlagLast) && upd;
+      if (mi) *mi = fin ? gmi[g] : 0u;
 #pragma unroll
       for (int c = 0; c < C; ++c) {
-        const uint32_t idx = (s * C + c) * GG + own + k;
-        vw[r][c] = fin ? gw[idx] : 0.f;
-        kc[r][c] = fin ? gkc[idx] : 0u;
+        const uint32_t idx = (s * C + c) * GG + g;
+        p[c] = !valid ? 0.f : !(word & kFlagFirst) ? gacc[idx] : has_ext ? gext[idx] : 0.f;
+        w[c] = fin ? gw[idx] : 0.f;
+        q[c] = fin ? gkc[idx] : 0u;
+      }
+    };
+#pragma unroll
+    for (int r = 0; r < KF; ++r) {
+      if constexpr (COL) {
+        load_slot(slot(r), prev[r], vw[r], kc[r], HO ? &mia[HO ? r : 0] : nullptr);
+      } else {
+        const int k = tid + r * T::BT;
+        const bool fin = upd && k < nint;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const uint32_t idx = (s * C + c) * GG + own + k;
+          vw[r][c] = fin ? gw[idx] : 0.f;
+          kc[r][c] = fin ? gkc[idx] : 0u;
+        }
       }
     }
     const bool more = s + 1 < s_end;
     float nu[T::NIT][C];
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
-      const bool ok = more && tid + r * T::BT < nval;
-      const uint32_t g = ok ? (sw[slr[r] & kSlotMask] & kNodeMask) : 0u;
+      const int l = slot(r);
+      const bool ok = more && (COL ? l >= 0 && sw[l] != kSlotEmpty : tid + r * T::BT < nval);
+      const uint32_t g = ok ? (sw[l] & kNodeMask) : 0u;
 #pragma unroll
       for (int c = 0; c < C; ++c) nu[r][c] = ok ? gu[((s + 1) * C + c) * GG + g] : 0.f;
     }
@@ -617,12 +662,66 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     // paths here, so that no slot's finish below waits for the stores of the
     // slots before it (stores count on the same counter, and the loads were
     // issued under branches the compiler's counting cannot follow)
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
-    // ---- finish every slot: its total is the face-summed result of its owner
+    // (not in the high-occupancy variant, whose later slots load in the finish
+    // loop: 0.5 % slower with the wait)
+    if (!HO) __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0) expcnt(7) lgkmcnt(15)
+    if constexpr (COL) {
+      // ---- finish every slot: its total joins the node's sum over the colours;
+      // the Newmark update at the last colour
+      const auto finish_slot = [&](int l, uint32_t o, const float(&p)[C], float(&w)[C], uint32_t(&q)[C], uint32_t mi) {
+        const uint32_t word = l >= 0 ? sw[l] : kSlotEmpty;
+        if (word == kSlotEmpty) return;
+        const bool first = (word & kFlagFirst) != 0, fin = (word & kFlagLast) && upd;
+#pragma unroll
+        for (int c = 0; c < C; ++c) {
+          const uint32_t idx = (s * C + c) * GG + (word & kNodeMask);
+          const float tot = sK[o + c * ND];
+          const float sum = first && !has_ext ? tot : p[c] + tot;
+          if (!fin) {
+            gacc[idx] = sum;
+            continue;
+          }
+          if (q3 && c == 2) continue;
+          const float a = __uint_as_float(mi) * sum;
+          float u = su[c * T::NTLP + l];
+          newmark(u, w[c], q[c], a, gdt, q3 && c == 0);
+          gu[idx] = u; gw[idx] = w[c]; gkc[idx] = q[c];
+          if (wap) gap[idx] = a;
+        }
+      };
+      // place of a lattice slot's total: the owner element's result
+      const auto place = [&](int l) -> uint32_t {
+        const int z = DIM == 3 ? l / T::LXYP : 0, rl = l - z * T::LXYP, y = rl / T::LXP, x = rl - y * T::LXP;
+        const int ea = min(x / N, ex - 1), eb = min(y / N, ey - 1), ec3 = DIM == 3 ? min(z / N, ez - 1) : 0;
+        return (ea + TX * (eb + TY * ec3)) * T::SKE + (x - ea * N) + n * ((y - eb * N) + n * (z - ec3 * N));
+      };
+#pragma unroll
+      for (int r = 0; r < KF; ++r) {
+        const int l = slot(r);
+        finish_slot(l, HO ? place(max(l, 0)) : slr[HO ? 0 : r] >> 16, prev[r], vw[r], kc[r], HO ? mia[HO ? r : 0] : mik[HO ? 0 : r]);
+      }
+      if constexpr (HO) {
+        constexpr int KB = 4;
+#pragma unroll 1
+        for (int r0 = KF; r0 < T::NIT; r0 += KB) {
+          float p[KB][C], w[KB][C];
+          uint32_t q[KB][C], mi[KB];
+          int ls[KB];
+#pragma unroll
+          for (int r = 0; r < KB; ++r) {
+            ls[r] = r0 + r < T::NIT ? slot(r0 + r) : -1;
+            load_slot(ls[r], p[r], w[r], q[r], &mi[r]);
+          }
+#pragma unroll
+          for (int r = 0; r < KB; ++r) finish_slot(ls[r], place(max(ls[r], 0)), p[r], w[r], q[r], mi[r]);
+        }
+      }
+    }
+    // ---- (partial results) finish every slot: its total is the face-summed result of its owner
     // element; this tile's partial result for a node shared with other tiles,
     // the Newmark update for any other
 #pragma unroll
-    for (int r = 0; r < T::NIT; ++r) {
+    for (int r = 0; r < (COL ? 0 : T::NIT); ++r) {
       const int k = tid + r * T::BT;
       if (k >= nval) continue;
       const uint32_t sv = again(slr[r]);
@@ -657,8 +756,8 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ>::BT))
     // own slots only: u of this shot has been read above
 #pragma unroll
     for (int r = 0; r < T::NIT; ++r) {
-      if (tid + r * T::BT >= nval) continue;
-      const int l = slr[r] & kSlotMask;
+      const int l = slot(r);
+      if (COL ? l < 0 : tid + r * T::BT >= nval) continue;
 #pragma unroll
       for (int c = 0; c < C; ++c) su[c * T::NTLP + l] = nu[r][c];
     }
@@ -746,14 +845,14 @@ int tile_kernel_shapes(int dim, int order, int physics, int *shapes, int max) {
 
 // Sets the dynamic-LDS limit of a kernel above 64 KiB and returns how many
 // of its workgroups one CU holds.
-template <int D, int N, int P, int X, int Y, int Z>
-static int prep_tile(int *per_cu) {
-  using S = TS<D, N, P, X, Y, Z>;
+template <int D, int N, int P, int X, int Y, int Z, int MODE>
+static int prep_one(int *per_cu) {
+  using S = TS<D, N, P, X, Y, Z, MODE == kTileColoursHigh>;
   const size_t shm = sizeof(float) * (size_t)S::LDS;
   if (shm > 160 * 1024) { set_error("tile does not fit in LDS"); return -1; }
-  const void *fn = (const void *)k_tile<D, N, P, X, Y, Z, false>;
+  const void *fn = (const void *)k_tile<D, N, P, X, Y, Z, false, MODE>;
   if (shm > 64 * 1024) {
-    const void *fns[2] = {fn, (const void *)k_tile<D, N, P, X, Y, Z, true>};
+    const void *fns[2] = {fn, (const void *)k_tile<D, N, P, X, Y, Z, true, MODE>};
     for (const void *f : fns) {
       hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm);
       if (e != hipSuccess) { set_error(std::string("tile LDS attribute: ") + hipGetErrorString(e)); return -2; }
@@ -766,36 +865,53 @@ static int prep_tile(int *per_cu) {
   return 0;
 }
 
-int tile_kernel_prepare(int dim, int order, int physics, const int *T, int *per_cu) {
+template <int D, int N, int P, int X, int Y, int Z>
+static int prep_tile(int mode, int *per_cu) {
+  if constexpr (P == SEM_ACOUSTIC)
+    if (mode == kTileColoursHigh) return prep_one<D, N, P, X, Y, Z, kTileColoursHigh>(per_cu);
+  return mode == kTileParts ? prep_one<D, N, P, X, Y, Z, kTileParts>(per_cu)
+                            : prep_one<D, N, P, X, Y, Z, kTileColours>(per_cu);
+}
+
+int tile_kernel_prepare(int dim, int order, int physics, const int *T, int mode, int *per_cu) {
   int rc = 1;
 #define TPR(D, N, X, Y, Z)                                                                  \
   if (rc == 1 && dim == D && order == N && same_shape(T, X, Y, D == 3 ? Z : 1))             \
-    rc = physics == SEM_ACOUSTIC ? prep_tile<D, N, 0, X, Y, Z>(per_cu)                      \
-                                 : prep_tile<D, N, 1, X, Y, Z>(per_cu);
+    rc = physics == SEM_ACOUSTIC ? prep_tile<D, N, 0, X, Y, Z>(mode, per_cu)                \
+                                 : prep_tile<D, N, 1, X, Y, Z>(mode, per_cu);
   SEM_TILE_KERNELS(TPR)
 #undef TPR
   if (rc == 1) { set_error("tile kernel not compiled for this order/shape"); return -1; }
   return rc;
 }
 
-template <int D, int N, int P, int X, int Y, int Z, bool DG>
-static int go_tile(const FusedArgs &a, hipStream_t st) {
-  using S = TS<D, N, P, X, Y, Z>;
-  hipLaunchKernelGGL((k_tile<D, N, P, X, Y, Z, DG>), dim3(a.nitems), dim3(S::BT), sizeof(float) * (size_t)S::LDS,
-                     st, a);
+template <int D, int N, int P, int X, int Y, int Z, bool DG, int MODE>
+static int go_mode(const FusedArgs &a, hipStream_t st) {
+  using S = TS<D, N, P, X, Y, Z, MODE == kTileColoursHigh>;
+  hipLaunchKernelGGL((k_tile<D, N, P, X, Y, Z, DG, MODE>), dim3(a.nitems), dim3(S::BT),
+                     sizeof(float) * (size_t)S::LDS, st, a);
   return 0;
 }
 
-int launch_tile(int dim, int order, int physics, const int *T, bool diag, const FusedArgs &a, hipStream_t st) {
+template <int D, int N, int P, int X, int Y, int Z, bool DG>
+static int go_tile(int mode, const FusedArgs &a, hipStream_t st) {
+  if constexpr (P == SEM_ACOUSTIC)
+    if (mode == kTileColoursHigh) return go_mode<D, N, P, X, Y, Z, DG, kTileColoursHigh>(a, st);
+  return mode == kTileParts ? go_mode<D, N, P, X, Y, Z, DG, kTileParts>(a, st)
+                            : go_mode<D, N, P, X, Y, Z, DG, kTileColours>(a, st);
+}
+
+int launch_tile(int dim, int order, int physics, const int *T, bool diag, int mode, const FusedArgs &a,
+                hipStream_t st) {
   if (a.nitems <= 0) return 0;
   int rc = 1;
 #define TLN(D, N, X, Y, Z)                                                                  \
   if (rc == 1 && dim == D && order == N && same_shape(T, X, Y, D == 3 ? Z : 1))             \
     rc = physics == SEM_ACOUSTIC                                                            \
-             ? (diag ? go_tile<D, N, 0, X, Y, Z, true>(a, st)                         \
-                     : go_tile<D, N, 0, X, Y, Z, false>(a, st))                       \
-             : (diag ? go_tile<D, N, 1, X, Y, Z, true>(a, st)                         \
-                     : go_tile<D, N, 1, X, Y, Z, false>(a, st));
+             ? (diag ? go_tile<D, N, 0, X, Y, Z, true>(mode, a, st)                         \
+                     : go_tile<D, N, 0, X, Y, Z, false>(mode, a, st))                       \
+             : (diag ? go_tile<D, N, 1, X, Y, Z, true>(mode, a, st)                         \
+                     : go_tile<D, N, 1, X, Y, Z, false>(mode, a, st));
   SEM_TILE_KERNELS(TLN)
 #undef TLN
   if (rc == 1) { set_error("tile kernel not compiled for this order/shape"); return -1; }

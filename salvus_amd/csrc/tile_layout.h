@@ -41,7 +41,8 @@ constexpr int round_to_residue(int a, int r, int m) { return a + (((r - a) % m) 
 // lattice slot of node (x, y, z) is x + LXP y + LXYP z), and per-element
 // strides of the lateral fluxes and the element results equal to NCOL modulo
 // 32 and 64, so that column thread t writes and reads bank (t + const) mod 32.
-// The slots in the tile tables are unpadded (x + LX y + LXY z).
+// The slots of the tiles' host tables are unpadded (x + LX y + LXY z), those of the
+// kernels' slot tables padded.
 template <int DIM, int N, int PHYS, int TX, int TY, int TZ, bool HO, bool PADDED>
 struct TSL {
   static constexpr int n = N + 1;
@@ -93,17 +94,19 @@ struct TSL {
   static constexpr int O_SK = ALIAS ? O_SW + NTLP : O_SF + EC * SFE;
   static constexpr int O_SE = ALIAS ? O_SF + EC * SFE : O_SK + E * SKE;
   // Register budget: 4 waves per SIMD (<= 128 VGPRs) with the finish
-  // inputs of every slot loaded ahead (up to KFMAX).  HO is the layout of a
-  // budget of 6 waves (<= 80 VGPRs, three slots ahead), which no kernel takes
-  // now: in one launch over all tiles the 4-wave budget was faster (3-D
-  // acoustic 64^3, 4x4x2 tiles: 203 us against 265 us with its spills).
+  // inputs of every slot loaded ahead (up to KFMAX); the high-occupancy
+  // variant HO of acoustic colour launches takes 6 (<= 80 VGPRs, a third
+  // workgroup per CU where LDS allows) and loads three slots per thread ahead.
+  // (In one launch over all tiles it was slower: 3-D acoustic 64^3, 4x4x2 tiles,
+  // 265 us against 203 us, with spills.)
   static constexpr int MINW = HO ? 6 : 4;
   static constexpr int KFR = HO ? 3 : KFMAX;
   static constexpr int KF = NIT < KFR ? NIT : KFR;
   static constexpr int O_SS = O_SE + E * NED;
   static constexpr int O_SD = O_SS + 4 * kTileMaxSrc + 1;
   // Threads take the tile words in node order (coalesced HBM accesses) and
-  // keep their words' slots in registers: no slot table in LDS.
+  // keep their words' slots in registers; HO takes them in lattice order, where
+  // the word's index is its slot.  No slot table in LDS in either.
   static constexpr bool SLOT_LDS = false;
   static constexpr int O_SL = O_SD + n * n;
   static constexpr int LDS = O_SL;

@@ -26,6 +26,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <map>
+#include <tuple>
 
 #include "sem_internal.h"
 
@@ -215,6 +217,80 @@ int build_tiles(sem_mesh *m, int Tx, int Ty, int Tz, TileSet &ts) {
   ts.T[0] = Tx; ts.T[1] = Ty; ts.T[2] = Tz;
   ts.valid = true;
   return 0;
+}
+
+// Nodes are renumbered tile-major by the tile that finishes them (the last
+// colour holding the node): each tile's nodes by position, its inside first and
+// then one run per lower/upper face, edge and corner, so that a tile's state and
+// each piece its neighbours share are contiguous.  The words of a tile come in
+// the order of their nodes, padding last.
+void build_colour_tiles(const sem_mesh *m, ColourTiles &ct, std::vector<uint16_t> &slot_of) {
+  const TileSet &ts = m->tiles;
+  const int dim = m->dim, N = m->order, LX = ts.T[0] * N + 1, LY = ts.T[1] * N + 1;
+  const int64_t NTL = ts.slots_per_tile, nt = ts.ntiles;
+  // per tile in lattice order: node in the other numbering (kSlotEmpty: none)
+  std::vector<uint32_t> lat(nt * NTL, kSlotEmpty);
+  std::vector<uint8_t> cmin(m->G, 255), cmax(m->G, 0), dir(m->G, 0);
+  for (int64_t t = 0; t < nt; ++t) {
+    const uint8_t c = (uint8_t)ts.info[t].colour;
+    for (int64_t k = t * NTL; k < t * NTL + ts.info[t].nval; ++k) {
+      const uint32_t g = ts.words[k] & kNodeMask;
+      lat[t * NTL + ts.slot_of[k]] = g;
+      cmin[g] = std::min(cmin[g], c);
+      cmax[g] = std::max(cmax[g], c);
+      if (ts.words[k] & kFlagDirichlet) dir[g] = 1;
+    }
+  }
+  // the slots of a tile of each extent by position, in slot order within it
+  std::map<std::tuple<int, int, int>, std::vector<int32_t>> by_place;
+  std::vector<int32_t> id(m->G, -1);
+  int32_t next = 0;
+  for (int64_t t = 0; t < nt; ++t) {
+    const TileInfo &ti = ts.info[t];
+    std::vector<int32_t> &place = by_place[std::make_tuple(ti.ex, ti.ey, ti.ez)];
+    if (place.empty()) {
+      const int last[3] = {ti.ex * N, ti.ey * N, dim == 3 ? ti.ez * N : -1};
+      std::vector<int32_t> cat(NTL);
+      for (int32_t s = 0; s < NTL; ++s) {
+        const int x[3] = {s % LX, (s / LX) % LY, s / (LX * LY)};
+        for (int a = 0, w = 1; a < dim; ++a, w *= 3) cat[s] += w * (x[a] == 0 ? 1 : x[a] == last[a] ? 2 : 0);
+        place.push_back(s);
+      }
+      std::stable_sort(place.begin(), place.end(), [&](int32_t a, int32_t b) { return cat[a] < cat[b]; });
+    }
+    for (int32_t s : place) {
+      const uint32_t g = lat[t * NTL + s];
+      if (g != kSlotEmpty && cmax[g] == ti.colour) id[g] = next++;
+    }
+  }
+  // words in the order of their nodes: mostly that of the tile before
+  ct.words.assign(nt * NTL, kSlotEmpty);
+  slot_of.assign(nt * NTL, 0);
+  std::vector<int32_t> order;  // slots, those without a node last
+  const auto key = [&](int64_t t, int32_t s) {
+    const uint32_t g = lat[t * NTL + s];
+    return g == kSlotEmpty ? m->G + s : (int64_t)id[g];
+  };
+  for (int64_t t = 0; t < nt; ++t) {
+    const auto before = [&](int32_t a, int32_t b) { return key(t, a) < key(t, b); };
+    if (order.empty())
+      for (int32_t s = 0; s < NTL; ++s) order.push_back(s);
+    if (!std::is_sorted(order.begin(), order.end(), before)) std::sort(order.begin(), order.end(), before);
+    for (int64_t k = 0; k < NTL; ++k) {
+      const uint32_t g = lat[t * NTL + order[k]];
+      slot_of[t * NTL + k] = (uint16_t)order[k];
+      if (g == kSlotEmpty) continue;
+      ct.words[t * NTL + k] = (uint32_t)id[g] | (cmin[g] == ts.info[t].colour ? kFlagFirst : 0u) |
+                              (cmax[g] == ts.info[t].colour ? kFlagLast : 0u) | (dir[g] ? kFlagDirichlet : 0u);
+    }
+  }
+  if (m->physics == SEM_ACOUSTIC) {
+    ct.words_lat.assign(nt * NTL, kSlotEmpty);
+    for (int64_t t = 0; t < nt; ++t)
+      for (int64_t k = 0; k < NTL; ++k) ct.words_lat[t * NTL + slot_of[t * NTL + k]] = ct.words[t * NTL + k];
+  }
+  ct.to_internal.resize(m->G);
+  for (int64_t g = 0; g < m->G; ++g) ct.to_internal[g] = id[ts.to_internal[g]];
 }
 
 }  // namespace sem
