@@ -586,7 +586,7 @@ static std::vector<WorkItem> element_items(sem_batch *b, const std::vector<int> 
 
 // Launches of one step: per kernel key the tiles of tiled groups or the
 // elements of the others, behind them the shared nodes of both; groups without
-// partial results one colour at a time.
+// partial results one colour at a time, each colour of all of them in one launch.
 static int build_plan(sem_batch *b) {
   // key = (lane, tile? | diagonal geometry << 1, dim, order, physics,
   // geometry mode, tile shape); SEM_TILE_GENERAL=1 keeps the general tile
@@ -702,16 +702,19 @@ static int build_plan(sem_batch *b) {
       SEM_TRY(upload(&l->d_items, items));
       SEM_TRY(upload(&l->d_elems, elems));
     } else {
-      for (int gi : kv.second) {
-        const sem_mesh *m = b->groups[gi].mesh;
-        L.group = gi;
-        for (int c = 0; c < m->ncol; ++c) {
-          L.colour = c;
-          L.first = m->col_start[c];
-          L.count = m->col_start[c + 1] - L.first;
-          L.nitems = (int)((L.count + b->epb - 1) / b->epb);
-          add(L);
+      int ncol = 0;
+      for (int gi : kv.second) ncol = std::max(ncol, b->groups[gi].mesh->ncol);
+      for (int c = 0; c < ncol; ++c) {
+        std::vector<WorkItem> items;
+        for (int gi : kv.second) {
+          const sem_mesh *m = b->groups[gi].mesh;
+          const int64_t end = c < m->ncol ? m->col_start[c + 1] : 0;
+          for (int64_t f = c < m->ncol ? m->col_start[c] : 0; f < end; f += b->epb)
+            items.push_back(WorkItem{gi, (int32_t)f, (int32_t)std::min<int64_t>(b->epb, end - f), 0, 0, 0, 0, 0, 0});
         }
+        L.colour = c;
+        L.nitems = (int)items.size();
+        SEM_TRY(upload(&add(L)->d_items, items));
       }
     }
   }
@@ -866,9 +869,6 @@ int enqueue_fused_step(sem_batch *b, int koff, int ku_only, int last) {
     a.elems = L.d_elems;
     a.tiles = L.d_tiles;
     a.nodes = L.d_nodes;
-    a.group = L.group;
-    a.first = L.first;
-    a.count = L.count;
     a.nitems = L.nitems;
     a.epb = b->epb;
     a.koff = koff;

@@ -124,10 +124,8 @@ struct LaunchSet {
   int nitems;
   int T[3];  // tile shape (tile kernel)
   int lane;  // stream lane (0: the batch stream, 1: the second stream)
-  int group;         // element kernel, one colour: its group and elements [first, first + count)
-  int64_t first, count;
-  WorkItem *d_items;   // element kernel, every element at once
-  int32_t *d_elems;
+  WorkItem *d_items;  // element kernel
+  int32_t *d_elems;   // and, every element at once, their elements
   TileItem *d_tiles;  // tile kernel
   NodeItem *d_nodes;  // shared-node kernel
 };

@@ -492,8 +492,8 @@ __device__ __forceinline__ void node_flux(const NodeCtx<DIM, N> &X, const NodeMa
 //     (Order2Newmark.cpp:68-115, w = v + dt/2 a_); for any other node each of
 //     its elements writes its partial result, which k_shared sums in the order
 //     of the elements' colours;
-//   colours (no A.elems: elements [first, first + count), one launch per
-//     colour): stored at a node's first colour, accumulated in HBM at the
+//   colours (no A.elems: one launch per colour over the items' elements or,
+//     without items, elements [first, first + count) of one group): stored at a node's first colour, accumulated in HBM at the
 //     next, finished at its last.  Taken where the partial results would take
 //     too much memory (elem_parts, and the allocation-free operator on meshes
 //     that keep none for it).
@@ -523,7 +523,7 @@ __global__ void __launch_bounds__(512) k_fused(FusedArgs A) {
   int gi = 0, s0 = 0, s1 = 1, nrec = 0, rec = 0, e0 = 0;
   bool active;
   int64_t e = 0;
-  if (colours) {
+  if (!A.items) {  // one group's colour
     const int64_t f = A.first + (int64_t)bid * A.epb;
     active = el < A.epb && f + el < A.first + A.count;
     if (active) e = f + el;
@@ -532,7 +532,7 @@ __global__ void __launch_bounds__(512) k_fused(FusedArgs A) {
   } else {
     const WorkItem W = glb(A.items)[bid];
     active = el < W.count;
-    if (active) e = glb(A.elems)[W.first + el];
+    if (active) e = colours ? W.first + el : glb(A.elems)[W.first + el];
     gi = W.group;
     s0 = W.s0;
     s1 = W.s1;

@@ -273,7 +273,8 @@ struct GroupDev {
 };
 
 // Work item of an element launch: shots [s0, s1) of `count` elements of one
-// group, in the launch's element list from `first` on.
+// group, in the launch's element list from `first` on; of a colour launch: every
+// shot (s1 = 0) of the elements at sorted positions from `first` on.
 struct WorkItem {
   int32_t group, first, count;
   uint16_t s0, s1;
@@ -342,10 +343,10 @@ struct ColourTiles {
 struct FusedArgs {
   const GroupDev *groups;
   const WorkItem *items;   // element kernel
-  const int32_t *elems;    // element kernel: the items' elements (null: one colour)
+  const int32_t *elems;    // element kernel: the items' elements (null: one colour, the items' sorted positions)
   const TileItem *tiles;   // tile kernel
   const NodeItem *nodes;   // shared-node kernel
-  int64_t first, count;    // element kernel, one colour: its elements of group `group`
+  int64_t first, count;    // element kernel, one colour without items: its elements of group `group`
   const float *u;          // accumulate-only pass on a caller's buffers (out set): input
   float *out;              // and result
   int32_t group;
