@@ -292,7 +292,11 @@ int64_t sem_reference_step_count(double duration, double dt, double *dt_out);
  * requests on the same mesh and dt whose step counts lie within a spread of
  * the largest (sem_server_set_grouping; default up to 4 shots, 10 %): they
  * form one multi-shot group that steps to its largest count, and each
- * request's seismograms are copied out at its own count.  Times are seconds
+ * request's seismograms are copied out at its own count.  The bytes charged to a
+ * request are those its group allocates for it; where the budget or the device
+ * does not hold that, a group on the fused path is set up in less memory (at
+ * most five arrays of a field, as a request is charged while it waits) with
+ * the same results.  Times are seconds
  * on the server's clock (sem_server_clock; 0 at creation).  path
  * SEM_PATH_PLAIN with max_active 1 is the one-shot-per-launch baseline (one
  * shot per group). */

@@ -101,17 +101,23 @@ static int weigh_group(sem_batch *b, int gi) {
   return 0;
 }
 
-int setup_group(sem_batch *b, int gi) {
+// Shared-node results of one plane (shot and component) of a group.
+static int64_t group_parts(const Group &g) {
+  return !g.parts ? 0 : g.tiled ? g.mesh->tiles.nparts : g.mesh->nparts;
+}
+
+int route_group(sem_batch *b, int gi) {
   Group &g = b->groups[gi];
   sem_mesh *m = g.mesh;
-  const int path = b->path;
-  int rc = weigh_group(b, gi);
-  if (rc) return rc;
+  const bool fused = b->path == SEM_PATH_FUSED;
+  SEM_TRY(weigh_group(b, gi));
   // tile kernel: 32-bit field offsets, 16-bit shot numbers and at most
   // kTileMaxSrc sources per tile
-  g.tiled = path == SEM_PATH_FUSED && m->tiles.valid &&
-            (uint64_t)m->c * (uint64_t)m->G * (uint64_t)g.S < (1ull << 32) && g.S < 65536;
-  if (g.tiled) {
+  g.tiled = fused && m->tiles.valid && (uint64_t)m->c * (uint64_t)m->G * (uint64_t)g.S < (1ull << 32) && g.S < 65536;
+  int64_t nsrc = 0;
+  for (int k : g.shots)
+    for (const SrcSpec &sp : b->shots[k].srcs) nsrc += sp.kind == 2 ? m->c : 1;
+  if (g.tiled && nsrc > kTileMaxSrc) {
     std::map<int64_t, int> per_tile;
     for (int sl = 0; sl < g.S && g.tiled; ++sl)
       for (auto &sp : b->shots[g.shots[sl]].srcs) {
@@ -126,14 +132,41 @@ int setup_group(sem_batch *b, int gi) {
         }
       }
   }
+  // partial results at shared nodes take at most an accumulator's memory in a
+  // lean group, else colour launches run on the accumulator; with both the
+  // results are the same
+  if (g.tiled) {
+    g.parts = g.lean ? m->tiles.nparts <= m->G : !(g.heavy || tile_occupancy(m));
+    if (!g.parts) SEM_TRY(ensure_colour_tiles(m));
+  } else {
+    if (fused && !g.lean) SEM_TRY(ensure_elem_parts(m));
+    g.parts = fused && m->elem_parts == 1 && g.S < 65536 && (!g.lean || m->nparts <= m->G);
+  }
+  g.routed = true;
+  return 0;
+}
+
+int64_t shot_bytes(const Group &g, const Shot &s, int64_t nsteps) {
+  const sem_mesh *m = g.mesh;
+  int64_t n = 4 * m->c * (g.parts ? 4 * m->G + group_parts(g) : 5 * m->G) + 8;  // fields, step counter
+  n += 4 * (int64_t)s.recs.size() * m->c * nsteps;
+  if (g.parts) n += (int64_t)s.recs.size() * ((int64_t)sizeof(TileRec) + 4 * m->nd);
+  for (const SrcSpec &p : s.srcs)
+    n += (p.kind == 2 ? m->c : 1) * (4 * nsteps + 4 * (int64_t)m->nd * m->c + (int64_t)sizeof(SrcDev));
+  return n;
+}
+
+int setup_group(sem_batch *b, int gi) {
+  Group &g = b->groups[gi];
+  sem_mesh *m = g.mesh;
+  const int path = b->path;
+  int rc = 0;
+  if (!g.routed) SEM_TRY(route_group(b, gi));
   const size_t len = (size_t)m->c * m->G * g.S;
   // u, w, a_, kc and the partial results at shared nodes (written before they
   // are read in each step) or the accumulator; kc = 0 is two bf16 zeros;
   // w = v + dt/2 a_ from the shot's initial v and a_
-  if (path == SEM_PATH_FUSED && !g.tiled) SEM_TRY(ensure_elem_parts(m));
-  g.parts = g.tiled ? !(g.heavy || tile_occupancy(m)) : path == SEM_PATH_FUSED && m->elem_parts == 1 && g.S < 65536;
-  if (g.tiled && !g.parts) SEM_TRY(ensure_colour_tiles(m));
-  const int64_t nparts = g.tiled ? m->tiles.nparts : m->nparts;
+  const int64_t nparts = group_parts(g);
   SEM_TRY(dalloc(&g.fields, g.parts ? 4 * len + (size_t)g.S * m->c * nparts : 5 * len, &g.bytes));
   std::vector<float> buf;
   const double half_dt = 0.5 * g.dt;
@@ -1028,6 +1061,13 @@ static void form_groups(sem_batch *b, int max_s) {
   }
 }
 
+static int set_up(sem_batch *b, int max_s, int epb) {
+  form_groups(b, max_s);
+  b->h_groups.resize(b->groups.size());
+  for (int gi = 0; gi < (int)b->groups.size(); ++gi) SEM_TRY(setup_group(b, gi));
+  return finalize_groups(b, epb);
+}
+
 static Shot *get_shot(sem_batch *b, int shot) {
   if (shot < 0 || shot >= (int)b->shots.size()) {
     set_error("shot index out of range");
@@ -1057,7 +1097,7 @@ static int read_space(sem_batch *b, const Group &g, size_t len, double **p, size
   *cap = b->read_cap;
   if (*cap) return 0;
   const size_t all = (size_t)g.mesh->c * g.mesh->G * g.S;
-  const size_t rest = g.parts ? (size_t)g.S * g.mesh->c * (g.tiled ? g.mesh->tiles.nparts : g.mesh->nparts) : all;
+  const size_t rest = g.parts ? (size_t)g.S * g.mesh->c * group_parts(g) : all;
   *p = reinterpret_cast<double *>(g.fields + 4 * all);
   *cap = rest / 2;
   if (*cap == 0) { set_error("no device memory for the field read-out"); return -3; }
@@ -1270,10 +1310,7 @@ int sem_batch_prepare(sem_batch *b, int path, int epb, int spg) {
     if (biggest > 1) {
       double best = 1e300;
       for (int cand = 1; cand <= std::min(biggest, 8); cand *= 2) {
-        form_groups(b, cand);
-        b->h_groups.resize(b->groups.size());
-        for (int gi = 0; gi < (int)b->groups.size() && !rc; ++gi) rc = setup_group(b, gi);
-        if (!rc) rc = finalize_groups(b, epb);
+        rc = set_up(b, cand, epb);
         const double t = rc ? -1 : time_steps(b, 3);
         batch_release(b);
         if (rc) return rc;
@@ -1287,11 +1324,7 @@ int sem_batch_prepare(sem_batch *b, int path, int epb, int spg) {
     }
   }
   // ---- grouping: shots sharing mesh, nsteps and dt
-  form_groups(b, max_s);
-  b->h_groups.resize(b->groups.size());
-  for (int gi = 0; gi < (int)b->groups.size(); ++gi)
-    if ((rc = setup_group(b, gi))) return fail(rc);
-  if ((rc = finalize_groups(b, epb))) return fail(rc);
+  if ((rc = set_up(b, max_s, epb))) return fail(rc);
   if (path == SEM_PATH_FUSED && epb <= 0) {
     bool any_elem = false;
     int nd_max = 1;
@@ -1321,11 +1354,7 @@ int sem_batch_prepare(sem_batch *b, int path, int epb, int spg) {
       }
       batch_release(b);
       b->path = path;
-      form_groups(b, max_s);
-      b->h_groups.resize(b->groups.size());
-      for (int gi = 0; gi < (int)b->groups.size(); ++gi)
-        if ((rc = setup_group(b, gi))) return fail(rc);
-      if ((rc = finalize_groups(b, best_epb))) return fail(rc);
+      if ((rc = set_up(b, max_s, best_epb))) return fail(rc);
     }
   }
   b->spg = max_s;

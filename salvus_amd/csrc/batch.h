@@ -69,6 +69,8 @@ struct Group {
   std::vector<int32_t> tile_src;  // tiled: tile of each source, ascending
   bool tiled = false;       // tile kernel; fields in the mesh's tile-major numbering
   bool parts = false;       // partial results at shared nodes; else colour launches
+  bool lean = false;        // set up in the least memory: at most five arrays of c*G*S
+  bool routed = false;      // route_group has decided
   bool heavy = false;       // of a batch whose tiles fill the chip often enough for colour launches
   int64_t *d_step = nullptr;  // device step counter
   float *d_seis = nullptr;    // seismograms of the group's shots
@@ -200,6 +202,11 @@ void free_tiles(sem_mesh *m);
 // batch.cpp
 // Position of DMPlex DOF entry i (= comp*G + g) in a group's field arrays.
 int64_t field_pos(const Group &g, int64_t i);
+// Decides the kernels of b->groups[gi] (tiled, parts) from its mesh, shots and
+// `lean`, and builds what its mesh lacks for them.
+int route_group(sem_batch *b, int gi);
+// Device bytes one shot takes in a group of that route and `nsteps` steps.
+int64_t shot_bytes(const Group &g, const Shot &s, int64_t nsteps);
 // Device state of b->groups[gi] from its shots (fields, sources, receivers);
 // fills b->h_groups[gi].
 int setup_group(sem_batch *b, int gi);

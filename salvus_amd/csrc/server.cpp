@@ -61,12 +61,10 @@ static double clock_of(const sem_server *s) {
   return std::chrono::duration<double>(std::chrono::steady_clock::now() - s->t0).count();
 }
 
-// Device bytes a request holds while active in a group of `nsteps` steps.
-static int64_t request_bytes(const sem_server *s, const Shot &sh, int64_t nsteps) {
+// Device bytes a request holds while active in group g of `nsteps` steps.
+static int64_t request_bytes(const sem_server *s, const Group &g, const Shot &sh, int64_t nsteps) {
   const sem_mesh *m = sh.mesh;
-  int64_t b = 5 * 4 * (int64_t)m->c * m->G + 8;
-  b += 4 * (int64_t)sh.recs.size() * m->c * nsteps;
-  b += (int64_t)sh.srcs.size() * (4 * nsteps + 4 * (int64_t)m->nd * m->c + (int64_t)sizeof(SrcDev));
+  int64_t b = shot_bytes(g, sh, nsteps);
   if (s->path == SEM_PATH_PLAIN) b += 2 * 4 * m->E * (int64_t)m->nd * m->c;  // gather/scatter scratch
   return b;
 }
@@ -203,7 +201,9 @@ int sem_server_submit(sem_server *s, sem_mesh *m, int64_t nsteps, double dt, dou
     SEM_TRY(locate(m, x.data(), &e, ref));
     r.shot.recs.push_back(x);
   }
-  r.bytes = request_bytes(s, r.shot, nsteps);
+  Group alone;  // the most a request needs at the least: five arrays
+  alone.mesh = m;
+  r.bytes = request_bytes(s, alone, r.shot, nsteps);
   if (r.bytes > s->budget) { set_error("request larger than the server's HBM budget"); return -1; }
   const int id = (int)s->reqs.size();
   s->reqs.push_back(std::move(r));
@@ -242,41 +242,52 @@ int sem_server_pump(sem_server *s, double *status) {
         nmax = hi;
         nmin = lo;
       }
-    auto bytes_of = [&](const std::vector<int> &ids, int64_t steps) {
-      int64_t t = 0;
-      for (int k : ids) t += request_bytes(s, s->reqs[k].shot, steps);
-      return t;
-    };
-    if (mem.size() > 1 && s->used + bytes_of(mem, nmax) > s->budget) {
-      mem.resize(1);  // the head alone, at its own step count
-      nmax = r.shot.nsteps;
-    }
-    if (s->used + bytes_of(mem, nmax) > s->budget) break;
-    Group g;
-    g.mesh = r.shot.mesh;
-    g.nsteps = nmax;
-    g.dt = r.shot.dt;
-    g.S = (int)mem.size();
-    for (int k : mem) {
-      b->shots.push_back(s->reqs[k].shot);
-      g.shots.push_back((int)b->shots.size() - 1);
-    }
-    b->groups.push_back(g);
-    const int gi = (int)b->groups.size() - 1;
-    const int rc = setup_group(b, gi);
-    if (rc) {
+    // The group, else the head alone at its own step count, each with its first
+    // choice of kernels, else in the least memory, as the budget and the device
+    // allow.  (What a mesh builds for a route is the mesh's own, as its other
+    // data: not part of a request.)
+    auto admit = [&](bool lean) {  // 1: set up, 0: does not fit now, < 0: error
+      Group g;
+      g.mesh = r.shot.mesh;
+      g.nsteps = nmax;
+      g.dt = r.shot.dt;
+      g.S = (int)mem.size();
+      g.lean = lean;
+      for (int k : mem) {
+        b->shots.push_back(s->reqs[k].shot);
+        g.shots.push_back((int)b->shots.size() - 1);
+      }
+      b->groups.push_back(g);
+      const int gi = (int)b->groups.size() - 1;
+      int rc = route_group(b, gi);
+      if (!rc) {
+        int64_t need = 0;
+        for (int k : mem) need += request_bytes(s, b->groups[gi], s->reqs[k].shot, nmax);
+        if (s->used + need <= s->budget && !(rc = setup_group(b, gi))) return 1;
+      }
       free_group(b->groups[gi]);
       b->groups.pop_back();
-      b->shots.resize(b->shots.size() - mem.size());  // admitted again later from the requests
+      b->shots.resize(b->shots.size() - mem.size());  // admitted again from the requests
       if ((int)b->h_groups.size() > gi) b->h_groups.resize(gi);
-      if (rc == -3) break;  // device memory short: retry after retirements
-      return rc;
+      if (rc == -3) (void)hipGetLastError();
+      return rc == -3 ? 0 : rc;
+    };
+    const bool fused = s->path == SEM_PATH_FUSED;
+    int got = admit(false);
+    if (!got && fused) got = admit(true);
+    if (!got && mem.size() > 1) {
+      mem.resize(1);
+      nmax = r.shot.nsteps;
+      got = admit(false);
+      if (!got && fused) got = admit(true);
     }
+    if (got < 0) return got;
+    if (!got) break;  // retry after retirements
     for (int k : mem) {
       Request &q = s->reqs[k];
       q.state = 1;
       q.t_admit = now;
-      q.bytes = request_bytes(s, q.shot, nmax);
+      q.bytes = request_bytes(s, b->groups.back(), q.shot, nmax);
       q.group_shots = (int)mem.size();
       s->used += q.bytes;
       ++s->nactive;

@@ -1,0 +1,68 @@
+"""Device memory of requests: a server charges what its groups allocate and
+admits what five arrays a shot allow, whatever its kernels would rather take;
+results are the same bit for bit."""
+import numpy as np
+import pytest
+
+from salvus_amd import sem
+from tests import problems as pb
+
+pytestmark = pytest.mark.gpu
+
+MIB = 1 << 20
+
+
+def problem(dim, physics, order, nel, distorted):
+    P = pb.make(dim, physics, nel, order=order, seed=6, distorted=distorted, nrec=2)
+    M = sem.Mesh(dim, order, physics, P["cells"], P["coords"], P["par"])
+    assert (M.ntiles == 0) == distorted
+    s = P["src"]
+    src = [dict(kind="force", loc=P["coords"][P["cells"][7 + 5 * k]].mean(0), amp=s["amp"], f0=s["f0"], t0=0.0, dir=s["dir"])
+           for k in range(4)]
+    P["recs"] = [P["coords"][P["cells"][e]].mean(0) for e in (8, 13, 18)]
+    return P, M, src
+
+
+def serve(P, M, src, nsteps, **kw):
+    S = sem.Server(block_steps=8, **kw)
+    ids = [S.submit(M, nsteps, P["dt"], [x], P["recs"]) for x in src]
+    st = S.pump()
+    S.drain()
+    return st, [S.result(i) for i in ids]
+
+
+@pytest.mark.parametrize("order,nel", [(1, 100), (2, 60)])
+def test_charged_bytes(order, nel):
+    """Deformed acoustic hexes of low order, whose partial results take eight and
+    three arrays: the charge covers the device memory gone after admission, up
+    to what the batch's tables, graph and allocation granularity take."""
+    import torch
+    P, M, src = problem(3, 0, order, nel, True)
+    serve(P, M, src, 8)  # what the mesh builds for itself is there
+    S = sem.Server(block_steps=8)
+    for x in src:
+        S.submit(M, 40, P["dt"], [x], P["recs"])
+    free = torch.cuda.mem_get_info()[0]
+    st = S.pump()
+    gone = free - torch.cuda.mem_get_info()[0]
+    assert st["active"] == 4 and gone > 4 * 5 * 4 * M.G  # more than the five arrays a shot
+    assert gone - 48 * MIB < st["bytes"] < gone + 48 * MIB
+    S.close()
+
+
+@pytest.mark.parametrize("dim,physics,order,nel,distorted", [
+    (3, 0, 1, 20, True), (3, 0, 2, 12, True), (3, 1, 4, 6, True), (2, 1, 1, 30, True), (3, 1, 2, 13, False)])
+def test_budget_of_five_arrays(dim, physics, order, nel, distorted):
+    """Three requests under a budget of three times their waiting charge: all
+    active at once, never past the budget, with the results of a server that
+    has all the memory it wants."""
+    P, M, src = problem(dim, physics, order, nel, distorted)
+    free, want = serve(P, M, src[:3], 24)
+    one = sem.Server(block_steps=8)
+    need = one.request(one.submit(M, 24, P["dt"], [src[0]], P["recs"]))["bytes"]
+    st, got = serve(P, M, src[:3], 24, hbm_budget=3 * need)
+    assert free["bytes"] > 3 * need  # the route of choice takes more
+    assert st["active"] == 3 and st["bytes"] <= 3 * need
+    for a, b in zip(got, want):
+        assert np.abs(b).max() > 0
+        np.testing.assert_array_equal(a, b)
