@@ -1056,16 +1056,31 @@ static void form_groups(sem_batch *b, int max_s) {
       g.dt = std::get<2>(kv.first);
       for (size_t j = k; j < std::min(list.size(), k + (size_t)max_s); ++j) g.shots.push_back(list[j]);
       g.S = (int)g.shots.size();
+      g.lean = b->lean;
       b->groups.push_back(g);
     }
   }
 }
 
-static int set_up(sem_batch *b, int max_s, int epb) {
+static int set_up_once(sem_batch *b, int max_s, int epb) {
   form_groups(b, max_s);
   b->h_groups.resize(b->groups.size());
   for (int gi = 0; gi < (int)b->groups.size(); ++gi) SEM_TRY(setup_group(b, gi));
   return finalize_groups(b, epb);
+}
+
+// Groups of up to max_s shots on the device; a batch that the device memory
+// does not hold with every group's first choice of kernels is set up again in
+// the least memory.
+static int set_up(sem_batch *b, int max_s, int epb) {
+  int rc = set_up_once(b, max_s, epb);
+  if (rc != -3 || b->lean || b->path != SEM_PATH_FUSED) return rc;
+  (void)hipGetLastError();
+  const int path = b->path;
+  batch_release(b);
+  b->path = path;
+  b->lean = true;
+  return set_up_once(b, max_s, epb);
 }
 
 static Shot *get_shot(sem_batch *b, int shot) {

@@ -169,6 +169,7 @@ struct sem_batch {
   int64_t kernel_launches = 0;
   std::vector<hipEvent_t> ev;  // timing: event pairs around timed kernels
   int64_t ev_launches = 0;       // kernel launches the event pairs cover
+  bool lean = false;             // groups set up in the least memory (Group::lean)
   std::vector<sem::CouplePair> couples;  // coupled fluid-solid shot pairs
   // Lanes: the groups split into parts of about equal work, each part's
   // launches on its own stream (lane 0: `stream`), forked from and

@@ -1,5 +1,6 @@
-"""Device memory of requests: a server charges what its groups allocate and
-admits what five arrays a shot allow, whatever its kernels would rather take;
+"""Device memory of requests and batches: a server charges what its groups
+allocate, admits what five arrays a shot allow whatever its kernels would
+rather take, and a batch that only fits in the least memory is set up in it;
 results are the same bit for bit."""
 import numpy as np
 import pytest
@@ -63,6 +64,37 @@ def test_budget_of_five_arrays(dim, physics, order, nel, distorted):
     st, got = serve(P, M, src[:3], 24, hbm_budget=3 * need)
     assert free["bytes"] > 3 * need  # the route of choice takes more
     assert st["active"] == 3 and st["bytes"] <= 3 * need
+    for a, b in zip(got, want):
+        assert np.abs(b).max() > 0
+        np.testing.assert_array_equal(a, b)
+
+
+def test_batch_in_the_least_memory():
+    """48 shots of 100^3 deformed order-1 hexes with 1400 MiB of the device left:
+    five arrays a shot (0.99 GB) fit, the twelve of partial results (2.37 GB) do
+    not."""
+    import torch
+    P, M, src = problem(3, 0, 1, 100, True)
+
+    def run():
+        B = sem.Batch()
+        for k in range(48):
+            B.add_shot(M, 12, P["dt"])
+            s = src[k % 4]
+            B.add_source(k, s["loc"], s["amp"], s["f0"], s["t0"], s["dir"])
+        B.prepare(sem.PATH_FUSED, 32, 4)
+        B.run(12)
+        out = [B.get_field(k, "u") for k in (0, 47)]
+        B.close()
+        return out
+
+    want = run()
+    hog = torch.empty(torch.cuda.mem_get_info()[0] - 1400 * MIB, dtype=torch.uint8, device="cuda")
+    try:
+        got = run()
+    finally:
+        del hog
+        torch.cuda.empty_cache()
     for a, b in zip(got, want):
         assert np.abs(b).max() > 0
         np.testing.assert_array_equal(a, b)
