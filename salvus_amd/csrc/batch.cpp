@@ -418,8 +418,7 @@ static void batch_release(sem_batch *b) {
   release_plan(b);
   dfree(b->d_groups);
   b->d_groups_cap = 0;
-  dfree(b->d_read);
-  b->read_cap = 0;
+  b->d_read = nullptr;
   dfree(b->d_uloc);
   dfree(b->d_aloc);
   b->uloc_cap = 0;
@@ -781,8 +780,19 @@ int finalize_groups(sem_batch *b, int epb_hint) {
   const size_t ng = b->groups.size();
   if (ng > b->d_groups_cap) {
     dfree(b->d_groups);
-    b->d_groups_cap = std::max<size_t>(std::max<size_t>(ng, 2 * b->d_groups_cap), 16);
-    SEM_TRY(dalloc(&b->d_groups, b->d_groups_cap));
+    b->d_read = nullptr;
+    const size_t cap = std::max<size_t>(std::max<size_t>(ng, 2 * b->d_groups_cap), 16);
+    const size_t table = (cap * sizeof(GroupDev) + 255) / 256 * 256;
+    b->d_groups_cap = 0;
+    unsigned char *p = nullptr;
+    if (b->read_len && dalloc(&p, table + b->read_len * sizeof(double)) == 0)
+      b->d_read = reinterpret_cast<double *>(p + table);
+    if (!p) {
+      (void)hipGetLastError();
+      SEM_TRY(dalloc(&p, table));
+    }
+    b->d_groups = reinterpret_cast<GroupDev *>(p);
+    b->d_groups_cap = cap;
   }
   if (ng)
     HIPCHK(hipMemcpyAsync(b->d_groups, b->h_groups.data(), ng * sizeof(GroupDev), hipMemcpyHostToDevice, b->stream));
@@ -1097,28 +1107,6 @@ static float *field_base(sem_batch *b, const Shot &s, int which) {
   return g.fields + (size_t)which * len;
 }
 
-// Device space of a field read-out, kept with the batch: one field, at most 32
-// MiB (a larger one is read in pieces); where no memory is left for it, the
-// group's own partial results or accumulator, which hold nothing between steps.
-static int read_space(sem_batch *b, const Group &g, size_t len, double **p, size_t *cap) {
-  size_t want = std::min<size_t>(len, (size_t)4 << 20);
-  if (b->read_cap < want) {
-    dfree(b->d_read);
-    b->read_cap = 0;
-    if (dalloc(&b->d_read, want) == 0) b->read_cap = want;
-    else (void)hipGetLastError();
-  }
-  *p = b->d_read;
-  *cap = b->read_cap;
-  if (*cap) return 0;
-  const size_t all = (size_t)g.mesh->c * g.mesh->G * g.S;
-  const size_t rest = g.parts ? (size_t)g.S * g.mesh->c * group_parts(g) : all;
-  *p = reinterpret_cast<double *>(g.fields + 4 * all);
-  *cap = rest / 2;
-  if (*cap == 0) { set_error("no device memory for the field read-out"); return -3; }
-  return 0;
-}
-
 extern "C" {
 
 int sem_batch_create(sem_batch **out, int device) {
@@ -1292,16 +1280,26 @@ int sem_shot_get_field(sem_batch *b, int shot, int which, double *vals) {
   }
   HIPCHK(hipSetDevice(b->device));
   Group &g = b->groups[s->group];
-  double *out = nullptr;
-  size_t cap = 0;
-  SEM_TRY(read_space(b, g, len, &out, &cap));
   const float *f = field_base(b, *s, which) + (size_t)s->slot * len;
   const float *ap = which == 1 ? field_base(b, *s, 2) + (size_t)s->slot * len : nullptr;  // v = w - dt/2 a_
-  for (size_t i = 0; i < len; i += cap) {
-    const size_t n = std::min(cap, len - i);
-    SEM_TRY(launch_read_field((int64_t)n, (int64_t)i, s->mesh->G, !g.tiled ? nullptr : g.parts ? s->mesh->d_to_int : s->mesh->ctiles.d_to_int, f, ap,
-                              0.5 * g.dt, out, b->stream));
-    HIPCHK(hipMemcpyAsync(vals + i, out, n * 8, hipMemcpyDeviceToHost, b->stream));
+  const double half_dt = 0.5 * g.dt;
+  if (!b->d_read) {  // the same on the host
+    std::vector<float> buf(len), abuf(ap ? len : 0);
+    HIPCHK(hipMemcpyAsync(buf.data(), f, len * 4, hipMemcpyDeviceToHost, b->stream));
+    if (ap) HIPCHK(hipMemcpyAsync(abuf.data(), ap, len * 4, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    for (size_t i = 0; i < len; ++i) {
+      const size_t k = field_pos(g, i);
+      vals[i] = ap ? (double)buf[k] - half_dt * (double)abuf[k] : (double)buf[k];
+    }
+    return 0;
+  }
+  const int32_t *to = !g.tiled ? nullptr : g.parts ? s->mesh->d_to_int : s->mesh->ctiles.d_to_int;
+  std::lock_guard<std::mutex> lock(b->read_mu);
+  for (size_t i = 0; i < len; i += b->read_len) {
+    const size_t n = std::min(b->read_len, len - i);
+    SEM_TRY(launch_read_field((int64_t)n, (int64_t)i, s->mesh->G, to, f, ap, half_dt, b->d_read, b->stream));
+    HIPCHK(hipMemcpyAsync(vals + i, b->d_read, n * 8, hipMemcpyDeviceToHost, b->stream));
   }
   HIPCHK(hipStreamSynchronize(b->stream));
   return 0;
@@ -1313,6 +1311,9 @@ int sem_batch_prepare(sem_batch *b, int path, int epb, int spg) {
   if (path != SEM_PATH_PLAIN && path != SEM_PATH_FUSED) { set_error("path"); return -1; }
   HIPCHK(hipSetDevice(b->device));
   b->path = path;
+  // one field, read out in pieces of at most 32 MiB
+  for (const Shot &s : b->shots) b->read_len = std::max(b->read_len, (size_t)s.mesh->c * s.mesh->G);
+  b->read_len = std::min<size_t>(b->read_len, (size_t)4 << 20);
   auto fail = [&](int r) { batch_release(b); return r; };
   int rc = 0;
   // ---- shots per group: given, 1 on the plain path, or autotuned: every

@@ -3,6 +3,7 @@
 #pragma once
 
 #include <array>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -154,8 +155,12 @@ struct sem_batch {
   std::vector<sem::GroupDev> h_groups;
   std::vector<sem::LaunchSet> launches;
   std::vector<sem::RecSet> recsets;
-  double *d_read = nullptr;  // field read-out: entries of one copy to the host
-  size_t read_cap = 0;
+  // field read-out: `read_len` entries (0: a server's batch) behind the group
+  // table, or none where the device had no memory left for them; one reader at a
+  // time
+  double *d_read = nullptr;
+  size_t read_len = 0;
+  std::mutex read_mu;
   float *d_uloc = nullptr, *d_aloc = nullptr;  // plain path scratch
   size_t uloc_cap = 0;
   hipGraphExec_t graph = nullptr;   // block_steps steps

@@ -51,6 +51,7 @@
 // so results are reproducible bit for bit.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstring>
 
 #include "sem_internal.h"
@@ -844,9 +845,14 @@ int tile_kernel_shapes(int dim, int order, int physics, int *shapes, int max) {
 }
 
 // Sets the dynamic-LDS limit of a kernel above 64 KiB and returns how many
-// of its workgroups one CU holds.
+// of its workgroups one CU holds; once per device (a batch's set-up asks several
+// times, at some 50 us each).
 template <int D, int N, int P, int X, int Y, int Z, int MODE>
 static int prep_one(int *per_cu) {
+  static std::atomic<int> known[64];
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) { set_error("device index"); return -1; }
+  if ((*per_cu = known[dev].load(std::memory_order_acquire)) > 0) return 0;
   using S = TS<D, N, P, X, Y, Z, MODE == kTileColoursHigh>;
   const size_t shm = sizeof(float) * (size_t)S::LDS;
   if (shm > 160 * 1024) { set_error("tile does not fit in LDS"); return -1; }
@@ -862,6 +868,7 @@ static int prep_one(int *per_cu) {
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, fn, S::BT, shm);
   if (e != hipSuccess) { set_error(std::string("tile occupancy: ") + hipGetErrorString(e)); return -2; }
   *per_cu = nb > 0 ? nb : 1;
+  known[dev].store(*per_cu, std::memory_order_release);
   return 0;
 }
 

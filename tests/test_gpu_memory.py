@@ -4,6 +4,7 @@ rather take, and a batch that only fits in the least memory is set up in it;
 results are the same bit for bit."""
 import numpy as np
 import pytest
+import torch
 
 from salvus_amd import sem
 from tests import problems as pb
@@ -37,7 +38,6 @@ def test_charged_bytes(order, nel):
     """Deformed acoustic hexes of low order, whose partial results take eight and
     three arrays: the charge covers the device memory gone after admission, up
     to what the batch's tables, graph and allocation granularity take."""
-    import torch
     P, M, src = problem(3, 0, order, nel, True)
     serve(P, M, src, 8)  # what the mesh builds for itself is there
     S = sem.Server(block_steps=8)
@@ -73,7 +73,6 @@ def test_batch_in_the_least_memory():
     """48 shots of 100^3 deformed order-1 hexes with 1400 MiB of the device left:
     five arrays a shot (0.99 GB) fit, the twelve of partial results (2.37 GB) do
     not."""
-    import torch
     P, M, src = problem(3, 0, 1, 100, True)
 
     def run():
