@@ -123,8 +123,9 @@ int sem_mesh_apply_stiffness(sem_mesh *mesh, int path, const float *u, float *ku
  * the reference; for callers that cannot allocate device memory: code under
  * HIP graph capture, tight serving loops).  u and ku are DEVICE buffers of
  * c x G floats in the DMPlex DOF order; ku = K u.  It allocates nothing:
- * a mesh whose partial results take at most 64 MiB keeps them, with the group
- * descriptor, from its creation on, and other meshes use a device array of the
+ * a mesh whose partial results take at most 64 MiB, and with their positions
+ * less than a thousandth of the device's free memory, keeps them with the group
+ * descriptor from its creation on, and other meshes use a device array of the
  * library, which each GPU holds until the process ends; a mesh whose largest element
  * colour needs more than 262,112 blocks (of up to 256 threads' worth of
  * elements: at order 4 in 3-D two elements each, 524,224 elements per colour)

@@ -129,6 +129,21 @@ static void bin_elements(sem_mesh *m) {
   each([&](int64_t b, int32_t e) { B.elem[cur[b]++] = e; });
 }
 
+// Temporary device space of one step: the mesh's while it is created, else its own.
+struct TempSpace {
+  unsigned char *p = nullptr;
+  bool own = false;
+  int get(sem_mesh *m, size_t bytes) {
+    own = bytes > m->temp_bytes;
+    if (own) return dalloc(&p, bytes);
+    p = m->d_temp;
+    return 0;
+  }
+  ~TempSpace() {
+    if (own) dfree(p);
+  }
+};
+
 // The gather map in the sorted (colour) order with its flags, built on the
 // device: the first and last colour of every node from one pass per colour
 // (a host loop over the element nodes took three times as long: 13 ms of the
@@ -136,8 +151,9 @@ static void bin_elements(sem_mesh *m) {
 static int upload_conn(sem_mesh *m) {
   const int64_t E = m->E, nd = m->nd;
   if (!m->d_conn) SEM_TRY(dalloc(&m->d_conn, E * nd, &m->bytes));
-  int32_t *d_raw = nullptr;  // one buffer: gather map, order, first and last colours, Dirichlet mask
-  SEM_TRY(dalloc(&d_raw, (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4)));
+  TempSpace temp;  // gather map, order, first and last colours, Dirichlet mask
+  SEM_TRY(temp.get(m, 4 * (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4)));
+  int32_t *d_raw = reinterpret_cast<int32_t *>(temp.p);
   int32_t *d_perm = d_raw + E * nd, *d_span = d_perm + E;
   uint8_t *d_dir = m->dirichlet.empty() ? nullptr : reinterpret_cast<uint8_t *>(d_span + 2 * m->G);
   int rc = 0;
@@ -155,7 +171,6 @@ static int upload_conn(sem_mesh *m) {
     rc = launch_conn_flags(m->col_start[c], m->col_start[c + 1] - m->col_start[c], (int)nd, c, d_perm, d_raw,
                            d_span, d_span + m->G, d_dir, m->d_conn, m->stream);
   if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "gather map");
-  dfree(d_raw);
   return rc;
 }
 
@@ -187,9 +202,10 @@ int sem::ensure_elem_parts(sem_mesh *m) {
   if (m->elem_parts >= 0) return 0;
   // elements per node; the nodes of each count, block of nodes by block
   const int nb = (int)((m->G + kClassNodes - 1) / kClassNodes);
-  int32_t *d_hits = nullptr;  // one buffer: elements per node, strides, counts, table
   std::vector<int32_t> count((size_t)nb * kNodeClasses);
-  SEM_TRY(dalloc(&d_hits, 2 * (size_t)m->G + count.size() + 3 * kNodeClasses));
+  TempSpace temp;  // elements per node, strides, counts, table
+  SEM_TRY(temp.get(m, 4 * (2 * (size_t)m->G + count.size() + 3 * kNodeClasses)));
+  int32_t *d_hits = reinterpret_cast<int32_t *>(temp.p);
   uint32_t *d_next = reinterpret_cast<uint32_t *>(d_hits), *d_stride = d_next + m->G;
   int32_t *d_count = d_hits + 2 * m->G;
   int rc = launch_fill_i32(m->G, d_hits, 0, m->stream);
@@ -197,7 +213,7 @@ int sem::ensure_elem_parts(sem_mesh *m) {
   if (!rc) rc = launch_class_count(m->G, d_hits, d_count, m->stream);
   if (!rc) rc = hip_check(hipMemcpyAsync(count.data(), d_count, count.size() * 4, hipMemcpyDeviceToHost, m->stream), "copy");
   if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
-  if (rc) { dfree(d_hits); return rc; }
+  if (rc) return rc;
   std::vector<int64_t> n(kNodeClasses, 0);  // elements per node -> nodes
   for (int b = 0; b < nb; ++b)
     for (int k = 0; k < kNodeClasses; ++k) {
@@ -219,13 +235,13 @@ int sem::ensure_elem_parts(sem_mesh *m) {
   }
   if ((parts > kMaxPartsPerNode * m->G && 4 * m->c * parts > kMaxSmallParts) || parts >= ((int64_t)1 << 32) ||
       n[kNodeClasses - 1]) {  // the last class: this many elements per node or more
-    dfree(d_hits);
     m->elem_parts = 0;
     return 0;
   }
-  rc = dalloc(&m->d_epos, (size_t)m->E * m->nd, &m->bytes);
-  if (!rc) rc = dalloc(&m->d_sh_node, (size_t)nodes, &m->bytes);
-  if (!rc) rc = hip_check(hipMemcpyAsync(d_count, count.data(), count.size() * 4, hipMemcpyHostToDevice, m->stream), "upload");
+  const size_t npos = (size_t)m->E * m->nd;
+  SEM_TRY(dalloc(&m->d_epos, npos + nodes, &m->bytes));  // one buffer: positions, shared nodes
+  m->d_sh_node = m->d_epos + npos;
+  rc = hip_check(hipMemcpyAsync(d_count, count.data(), count.size() * 4, hipMemcpyHostToDevice, m->stream), "upload");
   if (!rc) rc = hip_check(hipMemcpyAsync(d_count + count.size(), table.data(), table.size() * 4, hipMemcpyHostToDevice, m->stream), "upload");
   if (!rc) rc = launch_class_list(m->G, d_count, reinterpret_cast<const uint32_t *>(d_count + count.size()), d_next,
                                   d_stride, m->d_sh_node, m->stream);
@@ -233,10 +249,10 @@ int sem::ensure_elem_parts(sem_mesh *m) {
     rc = launch_elem_pos(m->col_start[c], m->col_start[c + 1] - m->col_start[c], m->nd, m->d_conn, d_stride,
                          d_next, m->d_epos, m->stream);
   if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
-  dfree(d_hits);
   if (rc) {
     dfree(m->d_epos);
-    dfree(m->d_sh_node);
+    m->d_sh_node = nullptr;
+    m->bytes -= (npos + nodes) * 4;
     return rc;
   }
   m->classes = classes;
@@ -486,8 +502,8 @@ static void mesh_free(sem_mesh *m) {
   dfree(m->d_tile_slot);
   dfree(m->d_sh_part);
   dfree(m->d_epos);
-  dfree(m->d_sh_node);
   dfree(m->d_apply_buf);
+  dfree(m->d_temp);
   dfree(m->d_telem);
   dfree(m->d_mi_int);
   dfree(m->d_to_int);
@@ -618,6 +634,9 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
   bin_elements(m);
   // device upload (sorted order)
   if ((rc = hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "stream"))) return fail(rc);
+  const size_t mass_bytes = 8 * ((size_t)E * m->nd + (size_t)m->G);  // the largest of the temporaries
+  if ((rc = dalloc(&m->d_temp, mass_bytes))) return fail(rc);
+  m->temp_bytes = mass_bytes;
   if ((rc = upload_conn(m))) return fail(rc);
   {
     std::vector<double> sv(E * nv * dim), sp(E * nv * npar);
@@ -651,9 +670,7 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
   }
   // FP64 mass: element contributions, colour-ordered assembly, reciprocal
   {
-    double *me = nullptr, *M = nullptr;
-    if ((rc = dalloc(&me, (size_t)E * m->nd))) return fail(rc);
-    if ((rc = dalloc(&M, (size_t)m->G))) { dfree(me); return fail(rc); }
+    double *me = reinterpret_cast<double *>(m->d_temp), *M = me + (size_t)E * m->nd;
     rc = launch_point_geometry(dim, order, physics, pointwise_mode(m), E, m->d_vtx, m->d_vpar, npar,
                                nullptr, me, m->stream);
     if (!rc) rc = launch_fill_f64(m->G, M, 0.0, m->stream);
@@ -663,15 +680,15 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
     if (!rc) rc = dalloc(&m->d_mi, (size_t)m->G, &m->bytes);
     if (!rc) rc = launch_reciprocal(m->G, M, m->d_mi, m->stream);
     if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "mass");
-    dfree(me);
-    dfree(M);
     if (rc) return fail(rc);
   }
   if (!affine && (rc = ensure_pointwise(m))) return fail(rc);
-  if ((rc = setup_tiles(m, nullptr))) return fail(rc);
   // what it keeps only makes the allocation-free operator faster: without the
   // memory for it the operator runs colour by colour
   if (setup_apply(m)) (void)hipGetLastError();
+  m->temp_bytes = 0;
+  dfree(m->d_temp);
+  if ((rc = setup_tiles(m, nullptr))) return fail(rc);
   *out = m;
   return 0;
 }

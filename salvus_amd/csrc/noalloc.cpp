@@ -6,7 +6,7 @@
 // everything else beforehand, so callers that may not call hipMalloc (graph
 // capture, tight serving loops) can use it.  It runs the element kernel on the
 // DMPlex-ordered fields directly:
-//  - on meshes whose partial results take at most 64 MiB, in two launches --
+//  - on meshes whose partial results are little (setup_apply), in two launches --
 //    every element, then the shared nodes -- with the descriptor, the partial
 //    results and the items kept with the mesh since its creation;
 //  - on larger ones colour by colour, with the descriptor and the step counter
@@ -75,13 +75,20 @@ int launched(const char *what) {
   return 0;
 }
 
+// A mesh keeps what the two launches need if that is little: at most 64 MiB of
+// partial results, and less than a thousandth of the device's free memory with
+// their positions, so that meshes whose owners never call the operator take no
+// memory that is missed.  (Creating a mesh takes 0.8 ms for it.)
 constexpr int64_t kMaxKeptParts = (int64_t)64 << 20;  // bytes
 
 }  // namespace
 
 int setup_apply(sem_mesh *m) {
-  // partial results number at most one per element node
+  // partial results number at most one per element node, their positions one
   if (4 * m->c * m->E * m->nd > kMaxKeptParts) return 0;
+  size_t free_bytes = 0, total = 0;
+  if (hipMemGetInfo(&free_bytes, &total) != hipSuccess || 4 * (m->c + 1) * m->E * m->nd > (int64_t)(free_bytes / 1024))
+    return 0;
   SEM_TRY(ensure_elem_parts(m));
   if (m->elem_parts != 1) return 0;
   const int epb = default_epb(m->nd);

@@ -511,7 +511,7 @@ struct sem_mesh {
   int elem_parts = -1;             // 1 built, 0 not taken (memory), -1 not decided
   int64_t nparts = 0;
   std::vector<sem::SharedClass> classes;
-  uint32_t *d_epos = nullptr, *d_sh_node = nullptr;
+  uint32_t *d_epos = nullptr, *d_sh_node = nullptr;  // (one buffer)
   // allocation-free operator on meshes small enough to keep partial results
   // for it (setup_apply): one buffer with the descriptor, the step counter (0),
   // the items and the partial results
@@ -533,6 +533,10 @@ struct sem_mesh {
   int32_t *d_to_int = nullptr;  // DMPlex DOF -> internal node
   sem::ColourTiles ctiles;  // built by the first group that takes colour launches
   bool tile_diag = false;  // every element's affine factors diagonal (axis-aligned lattice)
+  // while the mesh is created: one buffer for the steps' temporary data (an
+  // allocation and a release of some 100 us each for every one of them otherwise)
+  unsigned char *d_temp = nullptr;
+  size_t temp_bytes = 0;
   size_t bytes = 0;       // device bytes held (tile path included)
   size_t tile_bytes = 0;  // of which the tile path
 };

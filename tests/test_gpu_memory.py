@@ -2,16 +2,36 @@
 allocate, admits what five arrays a shot allow whatever its kernels would
 rather take, and a batch that only fits in the least memory is set up in it;
 results are the same bit for bit."""
+import ctypes as C
+from contextlib import contextmanager
+
 import numpy as np
 import pytest
-import torch
 
 from salvus_amd import sem
 from tests import problems as pb
+from tests.test_zz_no_alloc import Hip, noalloc
 
 pytestmark = pytest.mark.gpu
 
 MIB = 1 << 20
+
+
+def free_memory(hip):
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.L.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@contextmanager
+def only(left):
+    """All of the device's memory but `left` bytes held meanwhile."""
+    hip = Hip()
+    hog = hip.alloc(free_memory(hip) - left)
+    try:
+        yield
+    finally:
+        hip.L.hipFree(hog)
 
 
 def problem(dim, physics, order, nel, distorted):
@@ -43,9 +63,9 @@ def test_charged_bytes(order, nel):
     S = sem.Server(block_steps=8)
     for x in src:
         S.submit(M, 40, P["dt"], [x], P["recs"])
-    free = torch.cuda.mem_get_info()[0]
+    free = free_memory(Hip())
     st = S.pump()
-    gone = free - torch.cuda.mem_get_info()[0]
+    gone = free - free_memory(Hip())
     assert st["active"] == 4 and gone > 4 * 5 * 4 * M.G  # more than the five arrays a shot
     assert gone - 48 * MIB < st["bytes"] < gone + 48 * MIB
     S.close()
@@ -88,12 +108,23 @@ def test_batch_in_the_least_memory():
         return out
 
     want = run()
-    hog = torch.empty(torch.cuda.mem_get_info()[0] - 1400 * MIB, dtype=torch.uint8, device="cuda")
-    try:
+    with only(1400 * MIB):
         got = run()
-    finally:
-        del hog
-        torch.cuda.empty_cache()
     for a, b in zip(got, want):
         assert np.abs(b).max() > 0
         np.testing.assert_array_equal(a, b)
+
+
+def test_operator_keeps_nothing_that_is_missed():
+    """The allocation-free operator keeps its partial results with a mesh while
+    they are less than a thousandth of the free memory; without them it gives
+    the same bits."""
+    P = pb.make(3, 1, 16, seed=7)
+    u = np.random.default_rng(1).normal(size=(3, (16 * 4 + 1) ** 3)).astype(np.float32)
+    M = sem.Mesh(3, 4, 1, P["cells"], P["coords"], P["par"])
+    want = noalloc(M, u, Hip())
+    with only(4096 * MIB):
+        M2 = sem.Mesh(3, 4, 1, P["cells"], P["coords"], P["par"])
+        got = noalloc(M2, u, Hip())
+    assert M2.device_bytes < M.device_bytes - 4 * 16 ** 3 * 125
+    np.testing.assert_array_equal(got, want)

@@ -4,14 +4,13 @@ import threading
 
 import numpy as np
 import pytest
-import torch
 
 from salvus_amd import sem
 from tests import problems as pb
+from tests.test_gpu_memory import free_memory
+from tests.test_zz_no_alloc import Hip
 
 pytestmark = pytest.mark.gpu
-
-MIB = 1 << 20
 
 
 def batch(nel, shots, dim=3, distorted=False):
@@ -48,6 +47,6 @@ def test_threads_read_their_own_shot(distorted):
 
 def test_first_read_allocates_nothing():
     M, B, u = batch(30, 1)
-    free = torch.cuda.mem_get_info()[0]
+    free = free_memory(Hip())
     np.testing.assert_array_equal(B.get_field(0, "u"), u[0])
-    assert torch.cuda.mem_get_info()[0] == free
+    assert free_memory(Hip()) == free
