@@ -167,7 +167,25 @@ int setup_group(sem_batch *b, int gi) {
   // are read in each step) or the accumulator; kc = 0 is two bf16 zeros;
   // w = v + dt/2 a_ from the shot's initial v and a_
   const int64_t nparts = group_parts(g);
-  SEM_TRY(dalloc(&g.fields, g.parts ? 4 * len + (size_t)g.S * m->c * nparts : 5 * len, &g.bytes));
+  const size_t arrays = g.parts ? 4 * len + (size_t)g.S * m->c * nparts : 5 * len;
+  // The first group's allocation holds the batch's space for the field read-out
+  // too: one of its own would cost each batch 30 to 60 us, the first 300 to 600.
+  // An allocation above 64 MiB costs 0.2 ms more and its release 0.3 (fields
+  // of 2.3 M entries, 50 + 18 MB: 28.9 -> 29.5 ms for set-up, 470 steps and
+  // release), so one below it stays there with a smaller space.
+  const size_t at = (arrays + 63) / 64 * 64, most = ((size_t)64 << 20) / 4;
+  if (gi == 0 && b->read_len && !g.lean) {
+    const size_t room = at >= most ? b->read_len : std::max<size_t>((most - at) / 2, 128 << 10);
+    const size_t n = std::min(b->read_len, room);
+    if (dalloc(&g.fields, at + 2 * n, &g.bytes) == 0) {
+      b->d_read = reinterpret_cast<double *>(g.fields + at);
+      b->read_cap = n;
+    }
+  }
+  if (!g.fields) {
+    (void)hipGetLastError();  // (the read-out then runs on the host)
+    SEM_TRY(dalloc(&g.fields, arrays, &g.bytes));
+  }
   std::vector<float> buf;
   const double half_dt = 0.5 * g.dt;
   for (int which = 0; which < (g.parts ? 4 : 5); ++which) {
@@ -780,18 +798,9 @@ int finalize_groups(sem_batch *b, int epb_hint) {
   const size_t ng = b->groups.size();
   if (ng > b->d_groups_cap) {
     dfree(b->d_groups);
-    b->d_read = nullptr;
     const size_t cap = std::max<size_t>(std::max<size_t>(ng, 2 * b->d_groups_cap), 16);
-    const size_t table = (cap * sizeof(GroupDev) + 255) / 256 * 256;
     b->d_groups_cap = 0;
-    unsigned char *p = nullptr;
-    if (b->read_len && dalloc(&p, table + b->read_len * sizeof(double)) == 0)
-      b->d_read = reinterpret_cast<double *>(p + table);
-    if (!p) {
-      (void)hipGetLastError();
-      SEM_TRY(dalloc(&p, table));
-    }
-    b->d_groups = reinterpret_cast<GroupDev *>(p);
+    SEM_TRY(dalloc(&b->d_groups, cap));
     b->d_groups_cap = cap;
   }
   if (ng)
@@ -1081,10 +1090,10 @@ static int set_up_once(sem_batch *b, int max_s, int epb) {
 
 // Groups of up to max_s shots on the device; a batch that the device memory
 // does not hold with every group's first choice of kernels is set up again in
-// the least memory.
+// the least memory (and without the space for the read-out).
 static int set_up(sem_batch *b, int max_s, int epb) {
   int rc = set_up_once(b, max_s, epb);
-  if (rc != -3 || b->lean || b->path != SEM_PATH_FUSED) return rc;
+  if (rc != -3 || b->lean) return rc;
   (void)hipGetLastError();
   const int path = b->path;
   batch_release(b);
@@ -1283,6 +1292,7 @@ int sem_shot_get_field(sem_batch *b, int shot, int which, double *vals) {
   const float *f = field_base(b, *s, which) + (size_t)s->slot * len;
   const float *ap = which == 1 ? field_base(b, *s, 2) + (size_t)s->slot * len : nullptr;  // v = w - dt/2 a_
   const double half_dt = 0.5 * g.dt;
+  std::lock_guard<std::mutex> lock(b->read_mu);
   if (!b->d_read) {  // the same on the host
     std::vector<float> buf(len), abuf(ap ? len : 0);
     HIPCHK(hipMemcpyAsync(buf.data(), f, len * 4, hipMemcpyDeviceToHost, b->stream));
@@ -1295,9 +1305,8 @@ int sem_shot_get_field(sem_batch *b, int shot, int which, double *vals) {
     return 0;
   }
   const int32_t *to = !g.tiled ? nullptr : g.parts ? s->mesh->d_to_int : s->mesh->ctiles.d_to_int;
-  std::lock_guard<std::mutex> lock(b->read_mu);
-  for (size_t i = 0; i < len; i += b->read_len) {
-    const size_t n = std::min(b->read_len, len - i);
+  for (size_t i = 0; i < len; i += b->read_cap) {
+    const size_t n = std::min(b->read_cap, len - i);
     SEM_TRY(launch_read_field((int64_t)n, (int64_t)i, s->mesh->G, to, f, ap, half_dt, b->d_read, b->stream));
     HIPCHK(hipMemcpyAsync(vals + i, b->d_read, n * 8, hipMemcpyDeviceToHost, b->stream));
   }
@@ -1394,13 +1403,17 @@ int sem_batch_run(sem_batch *b, int64_t nsteps) {
   if (b->path == SEM_PATH_PLAIN) {
     const char *tg = getenv("SEM_TIME_KERNELS");
     b->timing = tg && tg[0] == '1';
-    for (int64_t k = 0; k < left; ++k) SEM_TRY(enqueue_plain_step(b));
+    for (int64_t k = 0; k < left; ++k) {
+      std::lock_guard<std::mutex> lock(b->read_mu);
+      SEM_TRY(enqueue_plain_step(b));
+    }
   } else {
     const char *tg = getenv("SEM_TIME_KERNELS");
     b->timing = tg && tg[0] == '1';
     const char *ng = getenv("SEM_NO_GRAPH");
     const bool graphs = !(ng && ng[0] == '1') && !b->timing;
     while (left > 0) {
+      std::lock_guard<std::mutex> lock(b->read_mu);  // no steps between the pieces of a read-out
       if (graphs) {  // full blocks, then one (cached) tail block
         const int k = (int)std::min<int64_t>(left, b->block_steps);
         SEM_TRY(capture_graph(b, k));

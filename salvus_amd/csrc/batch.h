@@ -155,11 +155,12 @@ struct sem_batch {
   std::vector<sem::GroupDev> h_groups;
   std::vector<sem::LaunchSet> launches;
   std::vector<sem::RecSet> recsets;
-  // field read-out: `read_len` entries (0: a server's batch) behind the group
-  // table, or none where the device had no memory left for them; one reader at a
-  // time
+  // field read-out: space for at most `read_len` entries (0: a server's batch),
+  // `read_cap` of them behind the first group's fields, or none where the device
+  // had no memory left for them; one reader, or a block of steps being enqueued,
+  // at a time
   double *d_read = nullptr;
-  size_t read_len = 0;
+  size_t read_len = 0, read_cap = 0;
   std::mutex read_mu;
   float *d_uloc = nullptr, *d_aloc = nullptr;  // plain path scratch
   size_t uloc_cap = 0;
