@@ -85,50 +85,6 @@ static bool is_affine(int dim, const double *v) {
   return true;
 }
 
-// Bins of about one element each over the mesh's bounding box, filled by a
-// counting sort in element order.
-static void bin_elements(sem_mesh *m) {
-  ElementBins &B = m->bins;
-  const int dim = m->dim;
-  double cells = 1;
-  for (int a = 0; a < dim; ++a) {
-    B.lo[a] = 1e300;
-    B.hi[a] = -1e300;
-    for (int64_t e = 0; e < m->E; ++e) {
-      B.lo[a] = std::min(B.lo[a], m->bbox[e * 2 * dim + a]);
-      B.hi[a] = std::max(B.hi[a], m->bbox[e * 2 * dim + dim + a]);
-    }
-    cells *= std::max(B.hi[a] - B.lo[a], 1e-300);
-  }
-  const double h = std::pow(cells / (double)m->E, 1.0 / dim);  // about an element
-  int64_t nb = 1;
-  for (int a = 0; a < dim; ++a) {
-    const double w = B.hi[a] - B.lo[a];
-    B.n[a] = (int)std::min(std::max(w / h, 1.0), 4.0 * std::pow((double)m->E, 1.0 / dim) + 1.0);
-    B.inv[a] = w > 0 ? B.n[a] / w : 0.0;
-    nb *= B.n[a];
-  }
-  auto each = [&](auto &&f) {
-    for (int64_t e = 0; e < m->E; ++e) {
-      const double *bb = &m->bbox[e * 2 * dim];
-      int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-      for (int a = 0; a < dim; ++a) {
-        lo[a] = B.at(a, bb[a]);
-        hi[a] = B.at(a, bb[dim + a]);
-      }
-      for (int z = lo[2]; z <= hi[2]; ++z)
-        for (int y = lo[1]; y <= hi[1]; ++y)
-          for (int x = lo[0]; x <= hi[0]; ++x) f(x + (int64_t)B.n[0] * (y + (int64_t)B.n[1] * z), (int32_t)e);
-    }
-  };
-  B.start.assign(nb + 1, 0);
-  each([&](int64_t b, int32_t) { ++B.start[b + 1]; });
-  for (int64_t b = 0; b < nb; ++b) B.start[b + 1] += B.start[b];
-  B.elem.resize(B.start[nb]);
-  std::vector<int64_t> cur(B.start.begin(), B.start.end() - 1);
-  each([&](int64_t b, int32_t e) { B.elem[cur[b]++] = e; });
-}
-
 // Temporary device space of one step: the mesh's while it is created, else its own.
 struct TempSpace {
   unsigned char *p = nullptr;
@@ -631,7 +587,7 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
     if (affine && !is_affine(dim, vx)) affine = false;
   }
   m->affine = affine;
-  bin_elements(m);
+  bin_elements(m->bins, dim, E, m->bbox.data());
   // device upload (sorted order)
   if ((rc = hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "stream"))) return fail(rc);
   const size_t mass_bytes = 8 * ((size_t)E * m->nd + (size_t)m->G);  // the largest of the temporaries
@@ -812,12 +768,9 @@ int sem_mesh_check_colouring(sem_mesh *m, int64_t *violations) {
 int sem::locate(const sem_mesh *m, const double *pt, int64_t *elem, double *ref) {
   const int dim = m->dim;
   const ElementBins &B = m->bins;
-  int64_t bin = 0;
   bool nan = false;  // in no bin and no box: every element is asked
-  for (int a = dim - 1; a >= 0; --a) {
-    nan = nan || std::isnan(pt[a]);
-    bin = bin * B.n[a] + B.at(a, pt[a]);
-  }
+  for (int a = 0; a < dim; ++a) nan = nan || std::isnan(pt[a]);
+  const int64_t bin = nan ? 0 : bin_of(B, dim, pt);
   const int64_t begin = nan ? 0 : B.start[bin], end = nan ? m->E : B.start[bin + 1];
   for (int64_t i = begin; i < end; ++i) {
     const int64_t e = nan ? i : B.elem[i];

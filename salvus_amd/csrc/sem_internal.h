@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "../../include/salvus_sem.h"
+#include "element_bins.h"
 #include "tile_layout.h"
 
 namespace sem {
@@ -465,20 +466,6 @@ int tile_kernel_prepare(int dim, int order, int physics, const int *T, int mode,
 // One workgroup per item (a.tiles).
 int launch_tile(int dim, int order, int physics, const int *T, bool diag, int mode, const FusedArgs &a,
                 hipStream_t st);
-
-// Bins over the elements' bounding boxes: the elements whose box meets bin b
-// are elem[start[b] .. start[b + 1]), ascending.
-struct ElementBins {
-  int n[3] = {1, 1, 1};
-  double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0}, inv[3] = {0, 0, 0};  // inv: bins per unit length
-  std::vector<int64_t> start;
-  std::vector<int32_t> elem;
-  // bin coordinate of x along axis a; monotone in x
-  int at(int a, double x) const {
-    const double f = (x - lo[a]) * inv[a];
-    return !(f > 0) ? 0 : f >= n[a] ? n[a] - 1 : (int)f;
-  }
-};
 
 }  // namespace sem
 
