@@ -194,8 +194,9 @@ int sem::ensure_elem_parts(sem_mesh *m) {
     m->elem_parts = 0;
     return 0;
   }
-  const size_t npos = (size_t)m->E * m->nd;
-  SEM_TRY(dalloc(&m->d_epos, npos + nodes, &m->bytes));  // one buffer: positions, shared nodes
+  // one buffer: positions, shared nodes (from a cache line's start on)
+  const size_t npos = ((size_t)m->E * m->nd + 63) / 64 * 64;
+  SEM_TRY(dalloc(&m->d_epos, npos + nodes, &m->bytes));
   m->d_sh_node = m->d_epos + npos;
   rc = hip_check(hipMemcpyAsync(d_count, count.data(), count.size() * 4, hipMemcpyHostToDevice, m->stream), "upload");
   if (!rc) rc = hip_check(hipMemcpyAsync(d_count + count.size(), table.data(), table.size() * 4, hipMemcpyHostToDevice, m->stream), "upload");
