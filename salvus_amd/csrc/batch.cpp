@@ -459,6 +459,17 @@ constexpr int kTileRounds = 2;
 // own behind the step.  With more shots or receivers in an item their samples
 // would be a serial chain (100 receivers along 500^2 elastic quads, loaded on
 // demand: 49 -> 55 us a step).
+//
+// Partial results of a launch of 3-D elastic tiles are stored past the caches
+// where they take a good part of the last-level cache (256 MB): smaller ones are
+// read back from it, larger ones only push out what the next tiles read.  MB of
+// them, us a step with stores through the caches, past them (order 4): 6, 24^3
+// hexes 37.0, 39.3; 15, 32^3 63.3, 68.3; 24, 4 shots of 24^3 101.6, 110.2; 29, 40^3
+// 111-115, 117; 51, 48^3 207-209, 211.5; 59, 4 of 32^3 252.3, 253.2; 102, 2 of 48^3
+// 419.8, 418.4; 119, 8 of 32^3 485.5, 482.5; 122, 64^3 466, 469; 245, 2 of 64^3
+// 965, 949; 490, 4 of 64^3 1831, 1788; order 3: 40^3 61.2, 66.1; order 2: 48^3 53.7,
+// 57.8.  (A branch at the store instead of a kernel mode: 0.4 % more on both sides.)
+constexpr int64_t kMaxCachedParts = (int64_t)96 << 20;
 static std::vector<TileItem> tile_items(sem_batch *b, const std::vector<int> &gis, int capacity, int waves) {
   int spw = 1;
   for (int gi : gis) spw = std::max(spw, b->groups[gi].S);
@@ -741,6 +752,12 @@ static int build_plan(sem_batch *b) {
       SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, kTileParts, &per_cu));
       const int waves = tile_kernel_info(L.dim, L.order, L.physics, L.T).threads / 64;
       const std::vector<TileItem> items = tile_items(b, kv.second, per_cu * cus, waves);
+      int64_t parts = 0;
+      for (int gi : kv.second) parts += 4 * b->groups[gi].S * L.c * group_parts(b->groups[gi]);
+      if (L.dim == 3 && L.physics == SEM_ELASTIC && parts > kMaxCachedParts) {
+        L.mode = kTilePartsPast;
+        SEM_TRY(tile_kernel_prepare(L.dim, L.order, L.physics, L.T, L.mode, &per_cu));
+      }
       L.nitems = (int)items.size();
       SEM_TRY(upload(&add(L)->d_tiles, items));
     } else if (!colours) {
@@ -784,7 +801,7 @@ static int build_plan(sem_batch *b) {
   for (const auto &L : b->launches)
     if (L.kind != kLaunchShared)
       per_step.insert(std::make_tuple((int)L.kind, (int)L.diag, L.dim, L.order, L.physics, L.gmode,
-                                      L.T[0] * 10000 + L.T[1] * 100 + L.T[2], L.colour, L.mode != kTileParts));
+                                      L.T[0] * 10000 + L.T[1] * 100 + L.T[2], L.colour, L.mode >= kTileColours));
   b->step_launches = (int)per_step.size();
   HIPCHK(hipStreamSynchronize(b->stream));
   return 0;

@@ -123,7 +123,7 @@ struct LaunchSet {
   int dim, order, physics, nd, c, colour;
   int gmode;  // geometry mode of the element kernel (kGeo*)
   bool diag;  // tile kernel: diagonal-geometry variant
-  int mode;   // tile kernel: kTileParts, kTileColours or kTileColoursHigh
+  int mode;   // tile kernel: kTile*
   int nitems;
   int T[3];  // tile shape (tile kernel)
   int lane;  // stream lane (0: the batch stream, 1: the second stream)

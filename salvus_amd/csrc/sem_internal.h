@@ -448,9 +448,10 @@ int launch_advance(int ngroups, const GroupDev *groups, int64_t k, hipStream_t s
 
 // ---------------------------------------------------------------- tile kernel (tile_kernels.hip)
 // Modes of the tile kernel: every tile in one launch, partial results at nodes
-// shared by tiles; one launch per tile colour, sums of shared nodes in HBM; the
-// same with more waves per SIMD (acoustic).
-enum { kTileParts, kTileColours, kTileColoursHigh };
+// shared by tiles; the same with these stored past the caches (3-D elastic); one
+// launch per tile colour, sums of shared nodes in HBM; the same with more waves per
+// SIMD (acoustic).
+enum { kTileParts, kTilePartsPast, kTileColours, kTileColoursHigh };
 int init_tile_tables(int device);
 struct TileKernelInfo {
   size_t lds_bytes;  // 0: no kernel compiled for this order and tile shape

@@ -167,14 +167,14 @@ __device__ __forceinline__ float p1_face(int v, float a, float b) {
 // diagonal (axis-aligned lattices), so the contractions keep their diagonal
 // terms only; the terms dropped are exact zeros, so results are those of the
 // general kernel.
-// MODE: partial results at shared nodes, or one launch per tile colour with the
-// sums of shared nodes in HBM (kTileColours; kTileColoursHigh: its acoustic
-// high-occupancy variant).
+// MODE: partial results at shared nodes (kTileParts; kTilePartsPast: stored past
+// the caches), or one launch per tile colour with the sums of shared nodes in HBM
+// (kTileColours; kTileColoursHigh: its acoustic high-occupancy variant).
 template <int DIM, int N, int PHYS, int TX, int TY, int TZ, bool DG, int MODE>
 __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ, MODE == kTileColoursHigh>::BT))
     __attribute__((amdgpu_waves_per_eu(TS<DIM, N, PHYS, TX, TY, TZ, MODE == kTileColoursHigh>::MINW)))
     k_tile(FusedArgs A) {
-  constexpr bool COL = MODE != kTileParts, HO = MODE == kTileColoursHigh;
+  constexpr bool HO = MODE == kTileColoursHigh, COL = MODE == kTileColours || HO;
   using T = TS<DIM, N, PHYS, TX, TY, TZ, HO>;
   constexpr int n = T::n, C = T::C, ND = T::ND, NL = T::NL;
   static_assert(HO || T::NIT == T::KF, "every slot's finish inputs are loaded ahead");
@@ -731,11 +731,8 @@ __global__ void __launch_bounds__((TS<DIM, N, PHYS, TX, TY, TZ, MODE == kTileCol
       for (int c = 0; c < C; ++c) {
         const float tot = sK[o + c * ND];
         if (k >= nint) {
-          // (3-D elastic tiles write up to half a field of partial results: past
-          // the caches, 64^3 elements x 4 shots 1847 -> 1812 us a step; smaller
-          // sets are read back from them)
           const gptr<float> at = gpart + (int64_t)(s * C + c) * PS + again(mik[r]);
-          if constexpr (DIM == 3 && C == 3) __builtin_nontemporal_store(tot, at);
+          if constexpr (MODE == kTilePartsPast) __builtin_nontemporal_store(tot, at);
           else *at = tot;
           continue;
         }
@@ -876,6 +873,8 @@ template <int D, int N, int P, int X, int Y, int Z>
 static int prep_tile(int mode, int *per_cu) {
   if constexpr (P == SEM_ACOUSTIC)
     if (mode == kTileColoursHigh) return prep_one<D, N, P, X, Y, Z, kTileColoursHigh>(per_cu);
+  if constexpr (D == 3 && P == SEM_ELASTIC)
+    if (mode == kTilePartsPast) return prep_one<D, N, P, X, Y, Z, kTilePartsPast>(per_cu);
   return mode == kTileParts ? prep_one<D, N, P, X, Y, Z, kTileParts>(per_cu)
                             : prep_one<D, N, P, X, Y, Z, kTileColours>(per_cu);
 }
@@ -904,6 +903,8 @@ template <int D, int N, int P, int X, int Y, int Z, bool DG>
 static int go_tile(int mode, const FusedArgs &a, hipStream_t st) {
   if constexpr (P == SEM_ACOUSTIC)
     if (mode == kTileColoursHigh) return go_mode<D, N, P, X, Y, Z, DG, kTileColoursHigh>(a, st);
+  if constexpr (D == 3 && P == SEM_ELASTIC)
+    if (mode == kTilePartsPast) return go_mode<D, N, P, X, Y, Z, DG, kTilePartsPast>(a, st);
   return mode == kTileParts ? go_mode<D, N, P, X, Y, Z, DG, kTileParts>(a, st)
                             : go_mode<D, N, P, X, Y, Z, DG, kTileColours>(a, st);
 }
