@@ -32,8 +32,9 @@ namespace {
 
 // Scratch: [0, 256) group descriptor, [256, 512) step counter.
 constexpr size_t kScratchBytes = 512;
-// Largest number of blocks a colour may need (an interface limit).
-constexpr int64_t kMaxItems = ((int64_t(4) << 20) - 512) / 16;
+// Largest number of blocks a colour may need: the entry point's documented
+// limit (the kernel itself takes any number a launch does).
+constexpr int64_t kMaxBlocks = 262112;
 static_assert(sizeof(GroupDev) <= 256, "group descriptor exceeds its scratch slot");
 
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
@@ -148,10 +149,10 @@ extern "C" int sem_mesh_apply_stiffness_noalloc(sem_mesh *m, const float *u, flo
   int64_t worst = 0;
   for (int c = 0; c < m->ncol; ++c)
     worst = std::max<int64_t>(worst, (m->col_start[c + 1] - m->col_start[c] + epb - 1) / epb);
-  if (worst > kMaxItems) {
+  if (worst > kMaxBlocks) {
     set_error("mesh too large for the allocation-free stiffness: a colour needs " +
-              std::to_string(worst) + " work items, at most " + std::to_string(kMaxItems) +
-              " are allowed (at most " + std::to_string(kMaxItems * epb) + " elements per colour)");
+              std::to_string(worst) + " blocks, at most " + std::to_string(kMaxBlocks) +
+              " are allowed (at most " + std::to_string(kMaxBlocks * epb) + " elements per colour)");
     return -1;
   }
   HIPCHK(hipSetDevice(m->device));
