@@ -100,15 +100,34 @@ struct TempSpace {
   }
 };
 
+// The Dirichlet flags of a gather map in place, for a device without the memory
+// that building it again takes.
+static int reflag_conn(sem_mesh *m) {
+  (void)hipGetLastError();
+  const size_t n = (size_t)m->E * m->nd, piece = (size_t)1 << 20;
+  std::vector<uint32_t> w(std::min(n, piece));
+  for (size_t i = 0; i < n; i += piece) {
+    const size_t k = std::min(piece, n - i);
+    HIPCHK(hipMemcpyAsync(w.data(), m->d_conn + i, k * 4, hipMemcpyDeviceToHost, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+    for (size_t j = 0; j < k; ++j)
+      w[j] = (w[j] & ~kFlagDirichlet) | (m->dirichlet[w[j] & kNodeMask] ? kFlagDirichlet : 0u);
+    HIPCHK(hipMemcpyAsync(m->d_conn + i, w.data(), k * 4, hipMemcpyHostToDevice, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+  }
+  return 0;
+}
+
 // The gather map in the sorted (colour) order with its flags, built on the
 // device: the first and last colour of every node from one pass per colour
 // (a host loop over the element nodes took three times as long: 13 ms of the
 // 102 ms set-up of 32^3 hexes).
 static int upload_conn(sem_mesh *m) {
   const int64_t E = m->E, nd = m->nd;
-  if (!m->d_conn) SEM_TRY(dalloc(&m->d_conn, E * nd, &m->bytes));
+  const bool built = m->d_conn != nullptr;
+  if (!built) SEM_TRY(dalloc(&m->d_conn, E * nd, &m->bytes));
   TempSpace temp;  // gather map, order, first and last colours, Dirichlet mask
-  SEM_TRY(temp.get(m, 4 * (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4)));
+  if (int rc = temp.get(m, 4 * (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4))) return built ? reflag_conn(m) : rc;
   int32_t *d_raw = reinterpret_cast<int32_t *>(temp.p);
   int32_t *d_perm = d_raw + E * nd, *d_span = d_perm + E;
   uint8_t *d_dir = m->dirichlet.empty() ? nullptr : reinterpret_cast<uint8_t *>(d_span + 2 * m->G);
