@@ -658,7 +658,13 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
     if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "mass");
     if (rc) return fail(rc);
   }
-  if (!affine && (rc = ensure_pointwise(m))) return fail(rc);
+  if (!affine && (rc = ensure_pointwise(m)) == -3) {  // the largest array: without the temporaries
+    (void)hipGetLastError();
+    m->temp_bytes = 0;
+    dfree(m->d_temp);
+    rc = ensure_pointwise(m);
+  }
+  if (rc) return fail(rc);
   // what it keeps only makes the allocation-free operator faster: without the
   // memory for it the operator runs colour by colour
   if (setup_apply(m)) (void)hipGetLastError();
