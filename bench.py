@@ -14,8 +14,9 @@ Workloads (--workload):
 A "step" advances every shot by one explicit Newmark time step (stiffness +
 sources + mass inverse + update + receivers).
 
-value        DOF-updates/s of the batched path: every shot in one set of tile
-             and shared-node kernel launches, hipGraph-captured step blocks, fields
+value        DOF-updates/s of the batched path: every shot in one set of kernel
+             launches (all tiles, then the nodes they share; large 3-D batches:
+             one tile launch per colour), hipGraph-captured step blocks, fields
              resident in HBM, K timed steps
 plain        the same shots through the plain one-shot-per-launch path
              (gather / stiffness / scatter / update kernels per shot)
@@ -62,14 +63,15 @@ def elem_floats(dim, physics):
     return ng + (2 ** dim) * kp
 
 
-def tile_bytes_per_step(M, S, dim, physics):
+def tile_bytes_per_step(M, S, dim, physics, colours=False):
     """Algorithmic HBM bytes of one step of one group on the tile kernel.
 
     per tile      : 4 B per lattice slot word + the elements' affine factors
                     and vertex material
     per shot      : u gather, 4c B per mesh slot (tile halos included); 4c B
                     written and read per partial result (one per tile holding
-                    a node shared by several); per node 4 B
+                    a node shared by several; with colour launches a node's
+                    sum, once less than it has tiles); per node 4 B
                     inverse mass + c (8 B read w, kc + 12 B write u, w, kc),
                     w = v + dt/2 a_ being the Newmark state the update reads
                     and kc the packed pair of bf16 Kahan compensations of u
@@ -77,8 +79,8 @@ def tile_bytes_per_step(M, S, dim, physics):
     """
     c = M.c
     per_tile = 4 * M.tile_slots + 4 * M.ntiles * M.tile_elems * elem_floats(dim, physics)
-    per_shot = (4 * c * M.tile_valid_slots + 4 * c * (M.tile_acc_reads + M.tile_acc_writes)
-                + M.G * (4 + 20 * c))
+    shared = 2 * (M.tile_valid_slots - M.G) if colours else M.tile_acc_reads + M.tile_acc_writes
+    per_shot = 4 * c * M.tile_valid_slots + 4 * c * shared + M.G * (4 + 20 * c)
     return per_tile + S * per_shot
 
 
@@ -222,7 +224,8 @@ def main():
     step_bytes = sum(element_bytes_per_step(M, k, dim, physics) for M, k in groups)
     per_launch_bytes = step_bytes / launches_per_step
     achieved = per_launch_bytes / avg_launch_s / 1e9
-    tile_launch_bytes = sum(tile_bytes_per_step(M, k, dim, physics) for M, k in groups) \
+    colours = cfg["tiled_groups"] > 0 and launches_per_step >= 2 ** dim
+    tile_launch_bytes = sum(tile_bytes_per_step(M, k, dim, physics, colours) for M, k in groups) \
         / launches_per_step
     tile_achieved = tile_launch_bytes / avg_launch_s / 1e9
     B.close()
@@ -268,7 +271,8 @@ def main():
                      "avg_launch_us": avg_launch_s * 1e6,
                      "launches_per_step": launches_per_step,
                      "launch_note": "a launch is every tile of one kernel shape and the shared-node "
-                                    "launch behind it (element kernel: one colour): with several "
+                                    "launch behind it, or one colour of its tiles (large 3-D "
+                                    "batches) or of the element kernel: with several "
                                     "lanes, its per-lane dispatches run side by side and count once",
                      "kernel_ms_per_step": kms / timing_steps},
     }

@@ -103,7 +103,6 @@ struct TempSpace {
 // The Dirichlet flags of a gather map in place, for a device without the memory
 // that building it again takes.
 static int reflag_conn(sem_mesh *m) {
-  (void)hipGetLastError();
   const size_t n = (size_t)m->E * m->nd, piece = (size_t)1 << 20;
   std::vector<uint32_t> w(std::min(n, piece));
   for (size_t i = 0; i < n; i += piece) {
@@ -659,7 +658,6 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
     if (rc) return fail(rc);
   }
   if (!affine && (rc = ensure_pointwise(m)) == -3) {  // the largest array: without the temporaries
-    (void)hipGetLastError();
     m->temp_bytes = 0;
     dfree(m->d_temp);
     rc = ensure_pointwise(m);

@@ -182,10 +182,7 @@ int setup_group(sem_batch *b, int gi) {
       b->read_cap = n;
     }
   }
-  if (!g.fields) {
-    (void)hipGetLastError();  // (the read-out then runs on the host)
-    SEM_TRY(dalloc(&g.fields, arrays, &g.bytes));
-  }
+  if (!g.fields) SEM_TRY(dalloc(&g.fields, arrays, &g.bytes));  // (the read-out then runs on the host)
   std::vector<float> buf;
   const double half_dt = 0.5 * g.dt;
   for (int which = 0; which < (g.parts ? 4 : 5); ++which) {
@@ -1111,7 +1108,6 @@ static int set_up_once(sem_batch *b, int max_s, int epb) {
 static int set_up(sem_batch *b, int max_s, int epb) {
   int rc = set_up_once(b, max_s, epb);
   if (rc != -3 || b->lean) return rc;
-  (void)hipGetLastError();
   const int path = b->path;
   batch_release(b);
   b->path = path;
@@ -1337,6 +1333,7 @@ int sem_batch_prepare(sem_batch *b, int path, int epb, int spg) {
   if (path != SEM_PATH_PLAIN && path != SEM_PATH_FUSED) { set_error("path"); return -1; }
   HIPCHK(hipSetDevice(b->device));
   b->path = path;
+  b->lean = false;
   // one field, read out in pieces of at most 32 MiB
   for (const Shot &s : b->shots) b->read_len = std::max(b->read_len, (size_t)s.mesh->c * s.mesh->G);
   b->read_len = std::min<size_t>(b->read_len, (size_t)4 << 20);

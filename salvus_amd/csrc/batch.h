@@ -23,6 +23,7 @@ inline int dalloc(T **p, size_t count, size_t *bytes = nullptr) {
     set_error(std::string("device allocation of ") + std::to_string(count * sizeof(T)) +
               " bytes failed: " + hipGetErrorString(e));
     *p = nullptr;
+    (void)hipGetLastError();  // the next launch's check would report it
     return -3;
   }
   if (bytes) *bytes += count * sizeof(T);

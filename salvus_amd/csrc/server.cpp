@@ -269,7 +269,6 @@ int sem_server_pump(sem_server *s, double *status) {
       b->groups.pop_back();
       b->shots.resize(b->shots.size() - mem.size());  // admitted again from the requests
       if ((int)b->h_groups.size() > gi) b->h_groups.resize(gi);
-      if (rc == -3) (void)hipGetLastError();
       return rc == -3 ? 0 : rc;
     };
     const bool fused = s->path == SEM_PATH_FUSED;
