@@ -100,18 +100,19 @@ struct TempSpace {
   }
 };
 
-// The Dirichlet flags of a gather map in place, for a device without the memory
-// that building it again takes.
-static int reflag_conn(sem_mesh *m) {
-  const size_t n = (size_t)m->E * m->nd, piece = (size_t)1 << 20;
-  std::vector<uint32_t> w(std::min(n, piece));
+// The Dirichlet flags of n words (node | flags, or kSlotEmpty) in place, a piece at
+// a time through the host.
+static int reflag_words(sem_mesh *m, uint32_t *d_words, size_t n, const std::vector<uint8_t> &dirichlet) {
+  const size_t piece = (size_t)1 << 20;
+  std::vector<uint32_t> words(std::min(n, piece));
   for (size_t i = 0; i < n; i += piece) {
     const size_t k = std::min(piece, n - i);
-    HIPCHK(hipMemcpyAsync(w.data(), m->d_conn + i, k * 4, hipMemcpyDeviceToHost, m->stream));
+    HIPCHK(hipMemcpyAsync(words.data(), d_words + i, k * 4, hipMemcpyDeviceToHost, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
     for (size_t j = 0; j < k; ++j)
-      w[j] = (w[j] & ~kFlagDirichlet) | (m->dirichlet[w[j] & kNodeMask] ? kFlagDirichlet : 0u);
-    HIPCHK(hipMemcpyAsync(m->d_conn + i, w.data(), k * 4, hipMemcpyHostToDevice, m->stream));
+      if (words[j] != kSlotEmpty)
+        words[j] = (words[j] & ~kFlagDirichlet) | (dirichlet[words[j] & kNodeMask] ? kFlagDirichlet : 0u);
+    HIPCHK(hipMemcpyAsync(d_words + i, words.data(), k * 4, hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipStreamSynchronize(m->stream));
   }
   return 0;
@@ -126,7 +127,8 @@ static int upload_conn(sem_mesh *m) {
   const bool built = m->d_conn != nullptr;
   if (!built) SEM_TRY(dalloc(&m->d_conn, E * nd, &m->bytes));
   TempSpace temp;  // gather map, order, first and last colours, Dirichlet mask
-  if (int rc = temp.get(m, 4 * (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4))) return built ? reflag_conn(m) : rc;
+  if (int rc = temp.get(m, 4 * (size_t)(E * nd + E + 2 * m->G + (m->G + 3) / 4)))
+    return built ? reflag_words(m, m->d_conn, (size_t)(E * nd), m->dirichlet) : rc;  // no memory for it: flags only
   int32_t *d_raw = reinterpret_cast<int32_t *>(temp.p);
   int32_t *d_perm = d_raw + E * nd, *d_span = d_perm + E;
   uint8_t *d_dir = m->dirichlet.empty() ? nullptr : reinterpret_cast<uint8_t *>(d_span + 2 * m->G);
@@ -263,6 +265,14 @@ static bool pick_tile(int dim, int order, int physics, int *T) {
 // (groups hold these buffers and read both in every step: a mask set later
 // acts on them too)
 static void free_colour_tiles(sem_mesh *m);
+static int reflag_colour_tiles(sem_mesh *m) {
+  const ColourTiles &ct = m->ctiles;
+  const size_t n = (size_t)m->tiles.ntiles * m->tiles.slots_per_tile;
+  std::vector<uint8_t> dirichlet(m->G);
+  for (int64_t g = 0; g < m->G; ++g) dirichlet[ct.to_internal[g]] = m->dirichlet[g];
+  SEM_TRY(reflag_words(m, ct.d_words, n, dirichlet));
+  return ct.d_words_lat ? reflag_words(m, ct.d_words_lat, n, dirichlet) : 0;
+}
 static int upload_tile_words(sem_mesh *m) {
   const TileSet &ts = m->tiles;
   if (!m->d_tile_words) SEM_TRY(dalloc(&m->d_tile_words, ts.words.size(), &m->tile_bytes));
@@ -281,18 +291,20 @@ static int upload_tile_words(sem_mesh *m) {
 // one extent and place in the box (inside, at a face, edge or corner) hold their
 // words in the same lattice order and share one table, which stays in the
 // caches: 4 bytes per slot less to read per tile and launch (one acoustic
-// shot, 10 of 73 KB at 4x4x2 tiles, 9 of 50 KB at 16x8).
+// shot, 10 of 73 KB at 4x4x2 tiles, 9 of 50 KB at 16x8).  Row r of slot_of, the
+// slots of the words in order, belongs to tile tiles[r] (empty: r itself).
 static std::vector<uint32_t> number_tile_slots(const sem_mesh *m, const std::vector<uint16_t> &slot_of,
-                                               std::vector<int32_t> &table) {
+                                               const std::vector<int32_t> &tiles, std::vector<int32_t> &table) {
   const TileSet &ts = m->tiles;
-  table.resize(ts.ntiles);
+  const int64_t rows = tiles.empty() ? ts.ntiles : (int64_t)tiles.size();
+  table.resize(rows);
   const TileKernelInfo k = tile_kernel_info(m->dim, m->order, m->physics, ts.T);
   const int N = m->order, n = m->n, LX = ts.T[0] * N + 1, LY = ts.T[1] * N + 1;
   const int64_t NTL = ts.slots_per_tile;
   std::vector<uint32_t> slot;
-  std::map<std::tuple<int, int, int>, std::vector<int32_t>> tables;  // per tile extent: the first tile of each table
-  for (int64_t t = 0; t < ts.ntiles; ++t) {
-    const TileInfo &ti = ts.info[t];
+  std::map<std::tuple<int, int, int>, std::vector<int32_t>> tables;  // per tile extent: the first row of each table
+  for (int64_t t = 0; t < rows; ++t) {
+    const TileInfo &ti = ts.info[tiles.empty() ? t : tiles[t]];
     std::vector<int32_t> &seen = tables[std::make_tuple(ti.ex, ti.ey, ti.ez)];
     const uint16_t *of = &slot_of[t * NTL];
     const auto same = [&](int32_t u) { return std::equal(of, of + NTL, &slot_of[u * NTL]); };
@@ -316,27 +328,66 @@ static std::vector<uint32_t> number_tile_slots(const sem_mesh *m, const std::vec
   return slot;
 }
 
-// Tables of the colour launches, built and uploaded once.
+// Numbering and words of the colour launches, built once.
 int sem::ensure_colour_tiles(sem_mesh *m) {
   std::lock_guard<std::mutex> lock(mesh_lazy);
   ColourTiles &ct = m->ctiles;
-  if (ct.valid) return 0;
-  std::vector<uint16_t> slot_of;
-  build_colour_tiles(m, ct, slot_of);
-  ct.slots = number_tile_slots(m, slot_of, ct.table);
+  if (ct.valid || ct.unfit) return 0;
+  const TileSet &ts = m->tiles;
+  const TileKernelInfo k = tile_kernel_info(m->dim, m->order, m->physics, ts.T);
+  const int ntl = (int)ts.slots_per_tile;
+  const size_t nwords = (size_t)ts.ntiles * ntl;
+  ColourTables c;
+  colour_tile_tables(m, c);
+  std::vector<int32_t> row;
+  const std::vector<uint32_t> slots = number_tile_slots(m, c.slot_of, c.example, row);
+  std::vector<ColourTile> tiles(ts.ntiles);
+  ct.table.resize(ts.ntiles);
+  for (int64_t t = 0; t < ts.ntiles; ++t) {
+    ct.table[t] = row[c.type[t]];
+    tiles[t] = ColourTile{c.type[t], ts.info[t].slots, ts.info[t].nval, c.first[t]};
+  }
   size_t bytes = 0;
-  auto up = [&](auto **dst, const auto &v) {
-    SEM_TRY(dalloc(dst, v.size(), &bytes));
-    if (v.empty()) return 0;
-    return hip_check(hipMemcpyAsync(*dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, m->stream), "upload");
+  int32_t bad = 0;
+  TempSpace temp;  // tiles, tables in both orders, flag
+  int rc = temp.get(m, tiles.size() * sizeof(ColourTile) + 8 * c.words.size() + 4);
+  ColourTile *d_tiles = reinterpret_cast<ColourTile *>(temp.p);
+  uint32_t *d_entries = reinterpret_cast<uint32_t *>(d_tiles + tiles.size()), *d_lat = d_entries + c.words.size();
+  int32_t *d_bad = reinterpret_cast<int32_t *>(d_lat + c.lat.size());
+  auto up = [&](void *dst, const auto &v) {
+    if (!rc) rc = hip_check(hipMemcpyAsync(dst, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice, m->stream), "upload");
   };
-  int rc = up(&ct.d_words, ct.words);
-  if (!rc) rc = up(&ct.d_words_lat, ct.words_lat);
-  if (!rc) rc = up(&ct.d_slot, ct.slots);
-  if (!rc) rc = up(&ct.d_to_int, ct.to_internal);
+  if (!rc) rc = dalloc(&ct.d_words, nwords, &bytes);
+  if (!rc && m->physics == SEM_ACOUSTIC) rc = dalloc(&ct.d_words_lat, nwords, &bytes);
+  if (!rc) rc = dalloc(&ct.d_slot, slots.size(), &bytes);
+  if (!rc) rc = dalloc(&ct.d_to_int, (size_t)m->G, &bytes);
   if (!rc) rc = dalloc(&ct.d_mi, (size_t)m->G, &bytes);
-  if (!rc) rc = launch_permute_f32(m->G, ct.d_to_int, m->d_mi, ct.d_mi, m->stream);
+  up(d_tiles, tiles);
+  up(d_entries, c.words);
+  up(d_lat, c.lat);
+  up(ct.d_slot, slots);
+  const int nx = ts.nt[0], nxy = ts.nt[0] * ts.nt[1];
+  int32_t *number = reinterpret_cast<int32_t *>(ct.d_mi);  // until the masses come
+  if (!rc) rc = launch_fill_i32(1, d_bad, 0, m->stream);
+  if (!rc) rc = launch_colour_words(ts.ntiles, ntl, nx, nxy, d_tiles, d_entries, ct.d_words, m->stream);
+  if (!rc && ct.d_words_lat) rc = launch_colour_words(ts.ntiles, ntl, nx, nxy, d_tiles, d_lat, ct.d_words_lat, m->stream);
+  if (!rc)
+    rc = launch_colour_numbers(ts.ntiles, ntl, ts.T[0] * m->order + 1, ts.T[1] * m->order + 1, k.lxp, k.lxyp, d_tiles, d_lat,
+                               m->d_tile_words, m->d_tile_slot, (uint32_t)ts.nown, (uint32_t)(ts.nown + ts.sh_n[0]),
+                               (uint32_t)(ts.nown + ts.sh_n[0] + ts.sh_n[1]), number, d_bad, m->stream);
+  if (!rc) rc = hip_check(hipMemcpyAsync(&bad, d_bad, 4, hipMemcpyDeviceToHost, m->stream), "copy");
   if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
+  if (rc || bad) {
+    free_colour_tiles(m);
+    ct.unfit = !rc;
+    return rc;
+  }
+  ct.to_internal.resize(m->G);
+  rc = launch_compose_i32(m->G, m->d_to_int, number, ct.d_to_int, m->stream);
+  if (!rc) rc = launch_permute_f32(m->G, ct.d_to_int, m->d_mi, ct.d_mi, m->stream);
+  if (!rc) rc = hip_check(hipMemcpyAsync(ct.to_internal.data(), ct.d_to_int, (size_t)m->G * 4, hipMemcpyDeviceToHost, m->stream), "copy");
+  if (!rc) rc = hip_check(hipStreamSynchronize(m->stream), "sync");
+  if (!rc && !m->dirichlet.empty()) rc = reflag_colour_tiles(m);
   if (rc) {
     free_colour_tiles(m);
     return rc;
@@ -402,7 +453,7 @@ int sem::upload_tiles(sem_mesh *m) {
   const int64_t E = (int64_t)ts.elem_order.size();
   {
     std::vector<int32_t> table;
-    m->tile_slots = number_tile_slots(m, ts.slot_of, table);
+    m->tile_slots = number_tile_slots(m, ts.slot_of, {}, table);
     for (int64_t t = 0; t < ts.ntiles; ++t) ts.info[t].slots = table[t];
   }
   SEM_TRY(upload_tile_words(m));
@@ -745,17 +796,7 @@ int sem_mesh_set_dirichlet(sem_mesh *m, const uint8_t *mask) {
       w = node | (dint[node] ? kFlagDirichlet : 0u);
     }
     SEM_TRY(upload_tile_words(m));
-    ColourTiles &ct = m->ctiles;
-    if (ct.valid) {
-      for (int64_t g = 0; g < m->G; ++g) dint[ct.to_internal[g]] = m->dirichlet[g];
-      for (auto *ws : {&ct.words, &ct.words_lat})
-        for (auto &w : *ws)
-          if (w != kSlotEmpty) w = (w & ~kFlagDirichlet) | (dint[w & kNodeMask] ? kFlagDirichlet : 0u);
-      HIPCHK(hipMemcpyAsync(ct.d_words, ct.words.data(), ct.words.size() * 4, hipMemcpyHostToDevice, m->stream));
-      if (ct.d_words_lat)
-        HIPCHK(hipMemcpyAsync(ct.d_words_lat, ct.words_lat.data(), ct.words_lat.size() * 4, hipMemcpyHostToDevice, m->stream));
-      HIPCHK(hipStreamSynchronize(m->stream));
-    }
+    if (m->ctiles.valid) SEM_TRY(reflag_colour_tiles(m));
   }
   return 0;
 }

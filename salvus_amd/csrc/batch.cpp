@@ -138,6 +138,7 @@ int route_group(sem_batch *b, int gi) {
   if (g.tiled) {
     g.parts = g.lean ? m->tiles.nparts <= m->G : !(g.heavy || tile_occupancy(m));
     if (!g.parts) SEM_TRY(ensure_colour_tiles(m));
+    g.parts = g.parts || m->ctiles.unfit;
   } else {
     if (fused && !g.lean) SEM_TRY(ensure_elem_parts(m));
     g.parts = fused && m->elem_parts == 1 && g.S < 65536 && (!g.lean || m->nparts <= m->G);

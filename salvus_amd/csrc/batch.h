@@ -195,7 +195,8 @@ int ensure_pointwise(sem_mesh *m);
 // Decides (once) whether the element kernel keeps partial results on this mesh
 // and builds their classes and positions.
 int ensure_elem_parts(sem_mesh *m);
-// Builds (once) what colour launches over the mesh's tiles need.
+// Builds (once) what colour launches over the mesh's tiles need, or marks them
+// unfit for it.
 int ensure_colour_tiles(sem_mesh *m);
 // noalloc.cpp: what the allocation-free operator keeps with a small mesh.
 int setup_apply(sem_mesh *m);

@@ -869,6 +869,48 @@ __global__ void k_permute_f32(int64_t n, const int32_t *__restrict__ to, const f
   if (i < n) dst[to[i]] = src[i];
 }
 
+// Colour launches: one block per tile (see colour_tile_tables).
+__global__ void __launch_bounds__(256) k_colour_words(int ntl, int nx, int nxy, const ColourTile *__restrict__ tiles,
+                                                      const uint32_t *__restrict__ entries,
+                                                      uint32_t *__restrict__ words) {
+  const int64_t t = blockIdx.x;
+  const uint32_t *e = entries + (int64_t)tiles[t].type * ntl;
+  for (int k = threadIdx.x; k < ntl; k += 256) {
+    const uint32_t w = e[k];
+    uint32_t out = kSlotEmpty;
+    if (w != kSlotEmpty) {
+      const int at = (w >> kRankBits) & 31;
+      const int64_t o = t + (at % 3 - 1) + nx * (at / 3 % 3 - 1) + (int64_t)nxy * (at / 9 - 1);
+      out = (tiles[o].first + (w & ((1u << kRankBits) - 1))) | (w & (kFlagFirst | kFlagLast));
+    }
+    words[t * ntl + k] = out;
+  }
+}
+__global__ void __launch_bounds__(256) k_colour_numbers(int ntl, int lx, int ly, int lxp, int lxyp,
+                                                        const ColourTile *__restrict__ tiles,
+                                                        const uint32_t *__restrict__ lat,
+                                                        const uint32_t *__restrict__ words,
+                                                        const uint32_t *__restrict__ slots, uint32_t class0,
+                                                        uint32_t class1, uint32_t class2, int32_t *__restrict__ number,
+                                                        int32_t *__restrict__ bad) {
+  const int64_t t = blockIdx.x;
+  const ColourTile T = tiles[t];
+  for (int k = threadIdx.x; k < T.nval; k += 256) {
+    const uint32_t node = words[t * ntl + k] & kNodeMask;
+    const int l = (int)(slots[(int64_t)T.slots * ntl + k] & kSlotMask);
+    const int z = l / lxyp, y = (l - z * lxyp) / lxp, x = l - z * lxyp - y * lxp;
+    const uint32_t w = lat[(int64_t)T.type * ntl + x + lx * (y + ly * z)];
+    const int shared = (int)(node >= class0) + (int)(node >= class1) + (int)(node >= class2);
+    if (w == kSlotEmpty || (int)((w >> kSharedShift) & 3) != shared) *bad = 1;
+    else if (w & kFlagLast) number[node] = (int32_t)(T.first + (w & ((1u << kRankBits) - 1)));
+  }
+}
+__global__ void k_compose_i32(int64_t n, const int32_t *__restrict__ from, const int32_t *__restrict__ number,
+                              int32_t *__restrict__ to) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) to[i] = number[from[i]];
+}
+
 // ------------------------------------------------------------------ plain path
 __device__ __forceinline__ void kahan_add(float &s, float &c, float x) {
   float y = x - c;
@@ -1189,6 +1231,26 @@ int launch_elem_pos(int64_t first, int64_t count, int nd, const uint32_t *conn, 
   if (count <= 0) return 0;
   k_elem_pos<<<nblocks(count * nd, 256), 256, 0, st>>>(first, count, nd, conn, stride, next, pos);
   return last_launch("element positions");
+}
+
+int launch_colour_words(int64_t ntiles, int ntl, int nx, int nxy, const ColourTile *tiles, const uint32_t *entries,
+                        uint32_t *words, hipStream_t st) {
+  if (ntiles <= 0) return 0;
+  k_colour_words<<<(unsigned)ntiles, 256, 0, st>>>(ntl, nx, nxy, tiles, entries, words);
+  return last_launch("colour words");
+}
+int launch_colour_numbers(int64_t ntiles, int ntl, int lx, int ly, int lxp, int lxyp, const ColourTile *tiles,
+                          const uint32_t *lat, const uint32_t *words, const uint32_t *slots, uint32_t class0,
+                          uint32_t class1, uint32_t class2, int32_t *number, int32_t *bad, hipStream_t st) {
+  if (ntiles <= 0) return 0;
+  k_colour_numbers<<<(unsigned)ntiles, 256, 0, st>>>(ntl, lx, ly, lxp, lxyp, tiles, lat, words, slots, class0, class1,
+                                                    class2, number, bad);
+  return last_launch("colour numbers");
+}
+int launch_compose_i32(int64_t n, const int32_t *from, const int32_t *number, int32_t *to, hipStream_t st) {
+  if (n <= 0) return 0;
+  k_compose_i32<<<nblocks(n, 256), 256, 0, st>>>(n, from, number, to);
+  return last_launch("compose");
 }
 
 int launch_permute_f32(int64_t n, const int32_t *to, const float *src, float *dst, hipStream_t st) {

@@ -311,6 +311,7 @@ struct TileSet {
   int64_t ntiles = 0, total_slots = 0;
   int64_t slots_per_tile = 0;        // (Tx N + 1)(Ty N + 1)(Tz N + 1)
   int elems_per_tile = 0;            // Tx Ty Tz
+  int nt[3] = {0, 0, 0};             // tiles along each axis (x fastest)
   std::vector<TileInfo> info;
   std::vector<uint32_t> words;       // per tile, own nodes then shared ones, each in node order:
                                      // internal node | Dirichlet flag, or kSlotEmpty
@@ -326,18 +327,36 @@ struct TileSet {
   std::vector<int32_t> elem_pos;     // element -> tile-order position
 };
 
-// The tables of the colour launches over the same tiles (build_colour_tiles), in
-// a node numbering of their own.
+// What the colour launches over the same tiles need, in a node numbering of
+// their own (words: node | flags, or kSlotEmpty).
 struct ColourTiles {
   bool valid = false;
-  std::vector<uint32_t> words;       // per tile, in node order: node | flags, or kSlotEmpty
-  std::vector<uint32_t> words_lat;   // acoustic: the same words in lattice order
+  bool unfit = false;                // neighbouring tiles do not share all their nodes: no such numbering
   std::vector<int32_t> table;        // slot table of each tile
-  std::vector<uint32_t> slots;
   std::vector<int32_t> to_internal;  // DMPlex DOF -> node
-  uint32_t *d_words = nullptr, *d_words_lat = nullptr, *d_slot = nullptr;
+  uint32_t *d_words = nullptr;       // per tile, in node order
+  uint32_t *d_words_lat = nullptr;   // acoustic: the same words in lattice order
+  uint32_t *d_slot = nullptr;
   float *d_mi = nullptr;
   int32_t *d_to_int = nullptr;
+};
+
+// Tables of every kind of tile neighbourhood (colour_tile_tables), a table per type of
+// slots_per_tile entries: rank among the nodes that the finishing tile finishes,
+// that tile's place (3 x 3 x 3 around this one), axes along which the node is
+// shared, kFlagFirst and kFlagLast; or kSlotEmpty.
+constexpr int kRankBits = 15, kSharedShift = 20;
+struct ColourTables {
+  std::vector<int32_t> type;      // of each tile
+  std::vector<uint32_t> first;    // first node that each tile finishes
+  std::vector<int32_t> example;   // a tile of each type
+  std::vector<uint32_t> words;    // in the words' order
+  std::vector<uint32_t> lat;      // in lattice order
+  std::vector<uint16_t> slot_of;  // lattice slot of each word
+};
+struct ColourTile {  // a tile as the kernels below read it
+  int32_t type, slots, nval;
+  uint32_t first;
 };
 
 // Kernel argument blocks (passed by value; recorded by graph capture).
@@ -431,6 +450,16 @@ int launch_class_list(int64_t G, const int32_t *first, const uint32_t *table, ui
 int launch_elem_pos(int64_t first, int64_t count, int nd, const uint32_t *conn, const uint32_t *stride,
                     uint32_t *next, uint32_t *pos, hipStream_t st);
 int launch_permute_f32(int64_t n, const int32_t *to, const float *src, float *dst, hipStream_t st);
+// Words of the colour launches from the tables of the tiles' types; the number
+// of every node from its number in `words`, whose nodes of one, two, four and eight
+// tiles begin at 0 and class0..2 (*bad is set where the tiles share others); and
+// to[i] = number[from[i]].
+int launch_colour_words(int64_t ntiles, int ntl, int nx, int nxy, const ColourTile *tiles, const uint32_t *entries,
+                        uint32_t *words, hipStream_t st);
+int launch_colour_numbers(int64_t ntiles, int ntl, int lx, int ly, int lxp, int lxyp, const ColourTile *tiles,
+                          const uint32_t *lat, const uint32_t *words, const uint32_t *slots, uint32_t class0,
+                          uint32_t class1, uint32_t class2, int32_t *number, int32_t *bad, hipStream_t st);
+int launch_compose_i32(int64_t n, const int32_t *from, const int32_t *number, int32_t *to, hipStream_t st);
 int launch_plain_gather(int64_t E, int nd, int C, int64_t G, const uint32_t *conn, const float *u,
                         float *uloc, hipStream_t st);
 int launch_plain_stiffness(int dim, int order, int physics, int gmode, int64_t E, int nd, int c,
@@ -549,6 +578,6 @@ inline int pointwise_mode(const sem_mesh *m) {
 }
 // Tiles a logically Cartesian mesh; 0 = tiled, 1 = not eligible.
 int build_tiles(sem_mesh *m, int Tx, int Ty, int Tz, TileSet &ts);
-// Numbering, words and lattice slot of each word (slot_of) for colour launches.
-void build_colour_tiles(const sem_mesh *m, ColourTiles &ct, std::vector<uint16_t> &slot_of);
+// Numbering and words of the colour launches by kinds of tiles.
+void colour_tile_tables(const sem_mesh *m, ColourTables &c);
 }  // namespace sem

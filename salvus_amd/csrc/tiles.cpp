@@ -24,6 +24,7 @@
 // its lattice slot (slot_of); sh_part holds the shared words' partial-result
 // positions.
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <map>
@@ -215,6 +216,7 @@ int build_tiles(sem_mesh *m, int Tx, int Ty, int Tz, TileSet &ts) {
   for (int64_t i = 0; i < ntiles * EPT; ++i)
     if (ts.elem_order[i] >= 0) ts.elem_pos[ts.elem_order[i]] = (int32_t)i;
   ts.T[0] = Tx; ts.T[1] = Ty; ts.T[2] = Tz;
+  for (int a = 0; a < 3; ++a) ts.nt[a] = (int)nt[a];
   ts.valid = true;
   return 0;
 }
@@ -224,73 +226,126 @@ int build_tiles(sem_mesh *m, int Tx, int Ty, int Tz, TileSet &ts) {
 // then one run per lower/upper face, edge and corner, so that a tile's state and
 // each piece its neighbours share are contiguous.  The words of a tile come in
 // the order of their nodes, padding last.
-void build_colour_tiles(const sem_mesh *m, ColourTiles &ct, std::vector<uint16_t> &slot_of) {
+//
+// All of it follows from a tile's place in the lattice: along an axis a node on
+// a face shared with the next tile is finished by the odd one of the two, so its
+// number is that tile's first plus its rank there, and ranks and order depend on the
+// kinds of a tile and its neighbours alone (extent, parity, faces shared): some
+// hundred tables at most, from which a device kernel writes every tile's words.
+// (Numbering slot by slot on the host took 0.3 s for 64^3 elastic hexes and 3 s
+// for 128^3 acoustic ones in the first large batch of a mesh.)
+void colour_tile_tables(const sem_mesh *m, ColourTables &c) {
   const TileSet &ts = m->tiles;
-  const int dim = m->dim, N = m->order, LX = ts.T[0] * N + 1, LY = ts.T[1] * N + 1;
-  const int64_t NTL = ts.slots_per_tile, nt = ts.ntiles;
-  // per tile in lattice order: node in the other numbering (kSlotEmpty: none)
-  std::vector<uint32_t> lat(nt * NTL, kSlotEmpty);
-  std::vector<uint8_t> cmin(m->G, 255), cmax(m->G, 0), dir(m->G, 0);
-  for (int64_t t = 0; t < nt; ++t) {
-    const uint8_t c = (uint8_t)ts.info[t].colour;
-    for (int64_t k = t * NTL; k < t * NTL + ts.info[t].nval; ++k) {
-      const uint32_t g = ts.words[k] & kNodeMask;
-      lat[t * NTL + ts.slot_of[k]] = g;
-      cmin[g] = std::min(cmin[g], c);
-      cmax[g] = std::max(cmax[g], c);
-      if (ts.words[k] & kFlagDirichlet) dir[g] = 1;
-    }
-  }
-  // the slots of a tile of each extent by position, in slot order within it
-  std::map<std::tuple<int, int, int>, std::vector<int32_t>> by_place;
-  std::vector<int32_t> id(m->G, -1);
-  int32_t next = 0;
-  for (int64_t t = 0; t < nt; ++t) {
-    const TileInfo &ti = ts.info[t];
-    std::vector<int32_t> &place = by_place[std::make_tuple(ti.ex, ti.ey, ti.ez)];
-    if (place.empty()) {
-      const int last[3] = {ti.ex * N, ti.ey * N, dim == 3 ? ti.ez * N : -1};
-      std::vector<int32_t> cat(NTL);
-      for (int32_t s = 0; s < NTL; ++s) {
-        const int x[3] = {s % LX, (s / LX) % LY, s / (LX * LY)};
-        for (int a = 0, w = 1; a < dim; ++a, w *= 3) cat[s] += w * (x[a] == 0 ? 1 : x[a] == last[a] ? 2 : 0);
-        place.push_back(s);
-      }
-      std::stable_sort(place.begin(), place.end(), [&](int32_t a, int32_t b) { return cat[a] < cat[b]; });
-    }
-    for (int32_t s : place) {
-      const uint32_t g = lat[t * NTL + s];
-      if (g != kSlotEmpty && cmax[g] == ti.colour) id[g] = next++;
-    }
-  }
-  // words in the order of their nodes: mostly that of the tile before
-  ct.words.assign(nt * NTL, kSlotEmpty);
-  slot_of.assign(nt * NTL, 0);
-  std::vector<int32_t> order;  // slots, those without a node last
-  const auto key = [&](int64_t t, int32_t s) {
-    const uint32_t g = lat[t * NTL + s];
-    return g == kSlotEmpty ? m->G + s : (int64_t)id[g];
+  const int N = m->order, NTL = (int)ts.slots_per_tile;
+  const int L[3] = {ts.T[0] * N + 1, ts.T[1] * N + 1, m->dim == 3 ? ts.T[2] * N + 1 : 1};
+  // kinds of tiles along each axis, and of a tile with the two next to it
+  struct Kind {
+    int last;              // last node
+    bool odd, low, high;   // parity; its faces are shared
+    bool operator<(const Kind &o) const { return std::tie(last, odd, low, high) < std::tie(o.last, o.odd, o.low, o.high); }
   };
-  for (int64_t t = 0; t < nt; ++t) {
-    const auto before = [&](int32_t a, int32_t b) { return key(t, a) < key(t, b); };
-    if (order.empty())
-      for (int32_t s = 0; s < NTL; ++s) order.push_back(s);
-    if (!std::is_sorted(order.begin(), order.end(), before)) std::sort(order.begin(), order.end(), before);
-    for (int64_t k = 0; k < NTL; ++k) {
-      const uint32_t g = lat[t * NTL + order[k]];
-      slot_of[t * NTL + k] = (uint16_t)order[k];
-      if (g == kSlotEmpty) continue;
-      ct.words[t * NTL + k] = (uint32_t)id[g] | (cmin[g] == ts.info[t].colour ? kFlagFirst : 0u) |
-                              (cmax[g] == ts.info[t].colour ? kFlagLast : 0u) | (dir[g] ? kFlagDirichlet : 0u);
+  std::vector<Kind> kinds[3];
+  std::vector<std::array<int, 3>> hoods[3];  // kinds of (previous, own, next) tile, -1: none
+  std::vector<int> hood[3];                  // of each tile of the axis
+  for (int a = 0; a < 3; ++a) {
+    const int n = ts.nt[a];
+    std::vector<int> kind(n);
+    std::map<Kind, int> kid;
+    std::map<std::array<int, 3>, int> hid;
+    for (int i = 0; i < n; ++i) {
+      const int64_t stride = a == 0 ? 1 : a == 1 ? ts.nt[0] : (int64_t)ts.nt[0] * ts.nt[1];
+      const TileInfo &ti = ts.info[i * stride];
+      const int e = a == 0 ? ti.ex : a == 1 ? ti.ey : ti.ez;
+      const Kind k{a < m->dim ? e * N : 0, (i & 1) != 0, i > 0, i < n - 1};
+      const auto it = kid.emplace(k, (int)kinds[a].size());
+      if (it.second) kinds[a].push_back(k);
+      kind[i] = it.first->second;
+    }
+    for (int i = 0; i < n; ++i) {
+      const std::array<int, 3> h{i > 0 ? kind[i - 1] : -1, kind[i], i < n - 1 ? kind[i + 1] : -1};
+      const auto it = hid.emplace(h, (int)hoods[a].size());
+      if (it.second) hoods[a].push_back(h);
+      hood[a].push_back(it.first->second);
     }
   }
-  if (m->physics == SEM_ACOUSTIC) {
-    ct.words_lat.assign(nt * NTL, kSlotEmpty);
-    for (int64_t t = 0; t < nt; ++t)
-      for (int64_t k = 0; k < NTL; ++k) ct.words_lat[t * NTL + slot_of[t * NTL + k]] = ct.words[t * NTL + k];
+  // ranks of the nodes a tile of each kind finishes (-1: another does), and how many
+  std::map<std::array<int, 3>, std::pair<std::vector<int32_t>, int32_t>> ranked;
+  const auto ranks = [&](const std::array<int, 3> &id) -> const std::pair<std::vector<int32_t>, int32_t> & {
+    auto &r = ranked[id];
+    if (!r.first.empty()) return r;
+    r.first.assign(NTL, -1);
+    int lo[3], hi[3], last[3];
+    for (int a = 0; a < 3; ++a) {
+      const Kind &k = kinds[a][id[a]];
+      last[a] = k.last;
+      lo[a] = k.low && !k.odd ? 1 : 0;
+      hi[a] = k.high && !k.odd ? k.last - 1 : k.last;
+    }
+    std::vector<std::pair<int, int32_t>> order;  // (position, slot)
+    for (int z = lo[2]; z <= hi[2]; ++z)
+      for (int y = lo[1]; y <= hi[1]; ++y)
+        for (int x = lo[0]; x <= hi[0]; ++x) {
+          const auto at = [&](int v, int a) { return v == 0 ? 1 : v == last[a] ? 2 : 0; };
+          order.emplace_back(at(x, 0) + 3 * at(y, 1) + 9 * at(z, 2), x + L[0] * (y + L[1] * z));
+        }
+    std::sort(order.begin(), order.end());
+    for (size_t i = 0; i < order.size(); ++i) r.first[order[i].second] = (int32_t)i;
+    r.second = (int32_t)order.size();
+    return r;
+  };
+  std::map<std::array<int, 3>, int32_t> tid;
+  c.type.resize(ts.ntiles);
+  c.first.resize(ts.ntiles);
+  uint32_t next = 0;
+  for (int64_t t = 0; t < ts.ntiles; ++t) {
+    const std::array<int, 3> id{hood[0][t % ts.nt[0]], hood[1][t / ts.nt[0] % ts.nt[1]],
+                                hood[2][t / ((int64_t)ts.nt[0] * ts.nt[1])]};
+    const std::array<int, 3> h[3] = {hoods[0][id[0]], hoods[1][id[1]], hoods[2][id[2]]};
+    c.first[t] = next;
+    next += (uint32_t)ranks({h[0][1], h[1][1], h[2][1]}).second;
+    const auto it = tid.emplace(id, (int32_t)tid.size());
+    c.type[t] = it.first->second;
+    if (!it.second) continue;
+    // a new neighbourhood: the tile that finishes each node, its rank there, the
+    // words' order (tiles in theirs, ranks)
+    const size_t o = c.words.size();
+    c.words.resize(o + NTL, kSlotEmpty);
+    c.lat.resize(o + NTL, kSlotEmpty);
+    std::vector<std::pair<uint32_t, int32_t>> order;  // (finishing tile and rank, slot)
+    for (int z = 0; z <= kinds[2][h[2][1]].last; ++z)
+      for (int y = 0; y <= kinds[1][h[1][1]].last; ++y)
+        for (int x = 0; x <= kinds[0][h[0][1]].last; ++x) {
+          const int v[3] = {x, y, z};
+          int at[3], d[3], shared = 0;
+          std::array<int, 3> owner;
+          bool starts = true, ends = true;
+          for (int a = 0; a < 3; ++a) {
+            const Kind &k = kinds[a][h[a][1]];
+            const bool low = k.low && v[a] == 0, high = k.high && v[a] == k.last;
+            d[a] = k.odd ? 0 : low ? -1 : high ? 1 : 0;
+            owner[a] = h[a][d[a] + 1];
+            at[a] = d[a] == 0 ? v[a] : d[a] < 0 ? kinds[a][owner[a]].last : 0;
+            shared += low || high;
+            starts = starts && !((low || high) && k.odd);
+            ends = ends && d[a] == 0;
+          }
+          const int32_t s = x + L[0] * (y + L[1] * z);
+          const uint32_t key = (uint32_t)(d[0] + 1 + 3 * (d[1] + 1) + 9 * (d[2] + 1)) << kRankBits |
+                               (uint32_t)ranks(owner).first[at[0] + L[0] * (at[1] + L[1] * at[2])];
+          order.emplace_back(key, s);
+          c.lat[o + s] = key | (uint32_t)shared << kSharedShift | (starts ? kFlagFirst : 0u) | (ends ? kFlagLast : 0u);
+        }
+    std::sort(order.begin(), order.end());
+    c.slot_of.resize(o + NTL, 0);
+    for (size_t k = 0; k < order.size(); ++k) {
+      c.words[o + k] = c.lat[o + order[k].second];
+      c.slot_of[o + k] = (uint16_t)order[k].second;
+    }
+    size_t k = order.size();
+    for (int32_t s = 0; s < NTL; ++s)
+      if (c.lat[o + s] == kSlotEmpty) c.slot_of[o + k++] = (uint16_t)s;
+    c.example.push_back((int32_t)t);
   }
-  ct.to_internal.resize(m->G);
-  for (int64_t g = 0; g < m->G; ++g) ct.to_internal[g] = id[ts.to_internal[g]];
 }
 
 }  // namespace sem
