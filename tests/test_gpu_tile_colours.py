@@ -80,3 +80,28 @@ def test_coupled_fluid(mode, monkeypatch):
     own test (FP64 oracle) with the fluid in colour launches."""
     monkeypatch.setenv("SEM_TILE_OCCUPANCY", mode)
     coupled.test_coupled_run(sem.PATH_FUSED, "straight", False, "f", False)
+
+
+@pytest.mark.parametrize("half", [False, True])
+def test_split_mesh_keeps_partial_results(half, monkeypatch):
+    """A box cut along a tile boundary (wholly, or up to its middle) is tiled, but
+    its tiles do not share all nodes of that face: no colour launches."""
+    box, at = (8, 8, 4), 4
+    cells, coords = meshgen.box_hex(*box, *[10.0 * n for n in box])
+    par = pb.vertex_material(3, 0, cells, coords, np.random.default_rng(1))
+    right = coords[cells].mean(1)[:, 0] > 10.0 * at
+    cut = np.flatnonzero((coords[:, 0] == 10.0 * at) & ((coords[:, 1] < 35.0) | (not half)))
+    twin = np.arange(len(coords))
+    twin[cut] = len(coords) + np.arange(len(cut))
+    cells = np.where(right[:, None], twin[cells], cells)
+    coords = np.vstack([coords, coords[cut]])
+    M = sem.Mesh(3, 4, 0, cells, coords, par)
+    assert M.ntiles == 2 * 2 * 2 and M.tile_shape == (4, 4, 2)
+    P = dict(cells=cells, coords=coords)
+    monkeypatch.setenv("SEM_TIME_KERNELS", "1")
+    n0, want = fields(M, P, 2, 9, None, range(2))
+    monkeypatch.setenv("SEM_TILE_OCCUPANCY", "normal")
+    n1, got = fields(M, P, 2, 9, None, range(2))
+    assert n0 == 9 and n1 == 9
+    for a, b in zip(got, want):
+        np.testing.assert_array_equal(a, b)
