@@ -86,6 +86,13 @@ static bool is_affine(int dim, const double *v) {
 }
 
 // Temporary device space of one step: the mesh's while it is created, else its own.
+// A mesh whose temporaries are small shares no buffer: its allocations come from
+// what the runtime keeps of released ones, and releasing them leaves more of that to
+// the first batch behind.  Creation and first pass, ms, with a shared buffer, without:
+// 100^2 acoustic quads (3 MB) 5.7, 5.3; 150x133 deformed elastic quads (7 MB) 10.1, 9.1;
+// 27x25x23 order-3 elastic hexes (11 MB) 27.4, 30.2; operator on 24x23x22 deformed
+// elastic hexes (18 MB) 10.9, 12.6; 31x30x29 deformed acoustic hexes (41 MB) 32.7, 35.1.
+constexpr size_t kMinShared = (size_t)8 << 20;
 struct TempSpace {
   unsigned char *p = nullptr;
   bool own = false;
@@ -661,8 +668,10 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
   // device upload (sorted order)
   if ((rc = hip_check(hipStreamCreateWithFlags(&m->stream, hipStreamNonBlocking), "stream"))) return fail(rc);
   const size_t mass_bytes = 8 * ((size_t)E * m->nd + (size_t)m->G);  // the largest of the temporaries
-  if ((rc = dalloc(&m->d_temp, mass_bytes))) return fail(rc);
-  m->temp_bytes = mass_bytes;
+  if (mass_bytes > kMinShared) {
+    if ((rc = dalloc(&m->d_temp, mass_bytes))) return fail(rc);
+    m->temp_bytes = mass_bytes;
+  }
   if ((rc = upload_conn(m))) return fail(rc);
   {
     std::vector<double> sv(E * nv * dim), sp(E * nv * npar);
@@ -696,7 +705,9 @@ int sem_mesh_create(sem_mesh **out, int device, int dim, int order, int physics,
   }
   // FP64 mass: element contributions, colour-ordered assembly, reciprocal
   {
-    double *me = reinterpret_cast<double *>(m->d_temp), *M = me + (size_t)E * m->nd;
+    TempSpace temp;
+    if ((rc = temp.get(m, mass_bytes))) return fail(rc);
+    double *me = reinterpret_cast<double *>(temp.p), *M = me + (size_t)E * m->nd;
     rc = launch_point_geometry(dim, order, physics, pointwise_mode(m), E, m->d_vtx, m->d_vpar, npar,
                                nullptr, me, m->stream);
     if (!rc) rc = launch_fill_f64(m->G, M, 0.0, m->stream);
